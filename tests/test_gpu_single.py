@@ -1,0 +1,56 @@
+"""GPU parity of the single-launch GEMVs at the edges of their tiling, bit
+for bit against the CPU oracle: row remainders, one tile and the last tile
+of an LDS batch, half tiles, and results stored over the activation."""
+import numpy as np
+import pytest
+from oracle import F16, F32, Q4_K, Q5_0, Q6_K, Q8_0
+from tmq import synth
+
+pytestmark = pytest.mark.gpu
+
+
+def bits(a):
+    return np.asarray(a, dtype=np.float32).view(np.uint32)
+
+
+# 64-column tiles: 1 (half), 2 (the second half full), 14, 128 = one LDS
+# batch, 129 (a half tile in a second batch), 200; rows 1, 8k, 8k + 1, 64k + 1
+@pytest.mark.parametrize("qt,rows,cols", [(F32, 1, 32), (Q8_0, 9, 96), (Q5_0, 65, 896), (Q4_K, 24, 8192),
+                                          (F16, 3, 8224), (Q5_0, 130, 12800), (Q6_K, 7, 4864)])
+def test_int16_edges(ctx, oracle, qt, rows, cols):
+    import tmq
+    print(f"[single] int16 type={qt} {rows}x{cols}", flush=True)
+    w = synth.gen_weights(qt, rows, cols, 41 + rows)
+    x = synth.gen_x(cols, 42 + cols)
+    t = ctx.upload(qt, rows, cols, w)
+    try:
+        acc, xs = ctx.partials_int16(t, x)
+        y = ctx.matmul_path(t, x, tmq.PATH_INT16)
+    finally:
+        t.free()
+    ye, te, _ = oracle.matmul_int16(qt, w, x, rows, cols)
+    assert xs == oracle.quantize_act(x)[1]
+    assert np.array_equal(acc, te)
+    assert np.array_equal(bits(y), bits(ye))
+
+
+@pytest.mark.parametrize("path", ["int16"])
+def test_result_over_activation(ctx, oracle, path):
+    """y written where x lies: every row still reads the whole x"""
+    import torch
+    import tmq
+    n = 896
+    w = synth.gen_weights(Q5_0, n, n, 51)
+    x = synth.gen_x(n, 52)
+    t = ctx.upload(Q5_0, n, n, w)
+    try:
+        for off in (0, 64, -64):
+            buf = torch.zeros(n + 128, dtype=torch.float32, device="cuda")
+            buf[64:64 + n] = torch.from_numpy(x)
+            torch.cuda.synchronize()
+            ctx.gemv_dev_path(t, {"int16": tmq.PATH_INT16}[path], buf.data_ptr() + 256, buf.data_ptr() + 256 + 4 * off)
+            ctx.sync()
+            y = buf[64 + off:64 + off + n].cpu().numpy()
+            assert np.array_equal(bits(y), bits(oracle.matmul_int16(Q5_0, w, x, n, n)[0])), off
+    finally:
+        t.free()

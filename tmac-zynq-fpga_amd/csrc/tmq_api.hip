@@ -431,6 +431,22 @@ TmqWork make_work(const tmq_tensor* t, const uint8_t* act, float* y, int64_t* ac
     return w;
 }
 
+// The activation a launch may read in every workgroup while others store
+// their results: x itself, or, where y or acc (acc_per int64 a row) lies over
+// it, a copy in the context's activation buffer (behind its x_scale).
+int own_x(tmq_ctx* ctx, const tmq_tensor* t, const float* x, const float* y, const int64_t* acc, size_t acc_per,
+          const float** out) {
+    const uintptr_t x0 = (uintptr_t)x, x1 = x0 + sizeof(float) * (size_t)t->dev.cols;
+    auto over = [&](const void* p, size_t n) { return p && (uintptr_t)p < x1 && x0 < (uintptr_t)p + n; };
+    *out = x;
+    if (!over(y, sizeof(float) * (size_t)t->dev.rows) && !over(acc, sizeof(int64_t) * acc_per * (size_t)t->dev.rows))
+        return 0;
+    float* c = (float*)((uint8_t*)ctx->act.p + 16);
+    HIP_TRY(hipMemcpyAsync(c, x, sizeof(float) * (size_t)t->dev.cols, hipMemcpyDeviceToDevice, ctx->stream));
+    *out = c;
+    return 0;
+}
+
 // run a GEMV with an int16 activation given on the host; int64 per-row
 // results returned on the host (tile API and PhaseB replay share this)
 int run_int16(tmq_ctx* ctx, const tmq_tensor* t, const int16_t* xq, std::vector<int64_t>& acc) {
@@ -859,18 +875,16 @@ int tmq_gemv_dev_path(tmq_ctx* ctx, const tmq_tensor* t, int path, const float* 
         LAUNCH_TRY(tmq_launch_gemv(w, ctx->stream));
         return 0;
     }
-    // INT16: weights quantised once per tensor, activation as every path does
+    // INT16: weights quantised once per tensor; the kernel quantises the
+    // activation and leaves x_scale at the start of the context's buffer
     rc = tmq_rt_prepare_int16(ctx, const_cast<tmq_tensor*>(t));
     if (!rc) rc = ctx->act.ensure(tmq_act_bytes(t->dev.cols));
     if (rc) return rc;
-    TmqActJobs jobs{};
-    jobs.count = 1;
-    jobs.j[0].x = x_dev;
-    jobs.j[0].act = (uint8_t*)ctx->act.p;
-    jobs.j[0].n = t->dev.cols;
-    LAUNCH_TRY(tmq_launch_act_prep(jobs, ctx->stream));
-    w = make_work(t, (const uint8_t*)ctx->act.p, y_dev, acc_dev);
+    w = make_work(t, nullptr, y_dev, acc_dev);
     w.path = TMQ_WPATH_INT16;
+    rc = own_x(ctx, t, x_dev, y_dev, acc_dev, (size_t)((t->dev.cols + 63) / 64), &w.xf);
+    if (rc) return rc;
+    w.xs_out = (float*)ctx->act.p;
     LAUNCH_TRY(tmq_launch_gemv(w, ctx->stream));
     return 0;
 }

@@ -116,13 +116,13 @@ struct TmqWork {
     const float* bias;   // may be null
     uint64_t* cand;      // Q8_0, engine GEMV: per-wave argmax candidate keys (may be null)
     int64_t* kacc;       // engine K-split: int64 row sums (zero before the launch)
-    float* xs_out;       // engine K-split: x_scale of the launch's activation
+    float* xs_out;       // engine K-split and the INT16 GEMV: x_scale of the launch's activation
     int32_t first_group;
     int32_t ngroups;     // workgroups of this GEMV (row groups x kc)
     int32_t kc;          // engine K-split: workgroups per row group (>= 1)
     int32_t resid;
     int32_t path;        // TMQ_WPATH_*: the type's own kernel, INT16 or FP32
-    const float* xf;     // FP32 path: the fp32 activation (act unused)
+    const float* xf;     // FP32 and INT16 GEMVs: the fp32 activation (act unused)
     // engine, kc = 1: fused SwiGLU.  The tensor holds ffn_gate and ffn_up
     // rows interleaved in groups of 32 (rows 64q..64q+31 = gate rows
     // 32q..32q+31, the next 32 = the same up rows); row j of the result,
