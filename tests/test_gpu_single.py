@@ -34,6 +34,23 @@ def test_int16_edges(ctx, oracle, qt, rows, cols):
     assert np.array_equal(bits(y), bits(ye))
 
 
+# 384 columns a batch: one block, one batch exactly, one block more, two
+# batches and a half; rows 1, 16k, 16k + 1, and past the lane-a-row bound
+@pytest.mark.parametrize("qt,rows,cols", [(F32, 1, 32), (Q8_0, 16, 384), (Q5_0, 17, 416), (F16, 40, 960), (Q4_K, 5, 1024),
+                                          (Q6_K, 33, 4864), (Q5_0, 65536, 32), (Q5_0, 65537, 64)])
+def test_fp32_edges(ctx, oracle, qt, rows, cols):
+    import tmq
+    print(f"[single] fp32 type={qt} {rows}x{cols}", flush=True)
+    w = synth.gen_weights(qt, rows, cols, 61 + rows)
+    x = synth.gen_x(cols, 62 + cols)
+    t = ctx.upload(qt, rows, cols, w)
+    try:
+        y = ctx.matmul_path(t, x, tmq.PATH_FP32)
+    finally:
+        t.free()
+    assert np.array_equal(bits(y), bits(oracle.matmul_fp32(qt, w, x, rows, cols)))
+
+
 @pytest.mark.parametrize("path", ["int16"])
 def test_result_over_activation(ctx, oracle, path):
     """y written where x lies: every row still reads the whole x"""

@@ -1836,75 +1836,116 @@ __global__ __launch_bounds__(64 * gemv_waves(FMT), FMT == kQ5_0M ? 8 : 1) void c
 // 32 exact elements of row r, columns j0..j0+31 (j0 % 32 == 0), evaluated as
 // read_tensor does: Q8_0 val*scale (:247), Q5_0 d*q (:322), Q6_K d*sc*q
 // (:360), Q4_K d*sc*q4 - dmin*m (:392), F32 as stored, F16 half->float.
-__device__ __forceinline__ void elems32(const TmqTensorDev& t, int r, int j0, float (&E)[32]) {
+// raw32 loads what they are made of, dec32 makes them.
+struct Raw32 {
+    uint4 v[8];
+    uint32_t a;
+};
+template <int FMT>
+__device__ __forceinline__ void raw32(const TmqTensorDev& t, int r, int j0, Raw32& k) {
     const size_t R = t.rows_pad;
-    if (t.type == kQ8_0) {
+    if constexpr (FMT == kQ8_0) {
         const int b = j0 >> 5;
-        const uint4 v0 = ld16(t.pa + p16(b, 0, 2, R, r)), v1 = ld16(t.pa + p16(b, 1, 2, R, r));
-        const float d = h2f(ld2(t.pd + ((size_t)b * R + r) * 2));
+        k.v[0] = ld16(t.pa + p16(b, 0, 2, R, r));
+        k.v[1] = ld16(t.pa + p16(b, 1, 2, R, r));
+        k.a = ld2(t.pd + ((size_t)b * R + r) * 2);
+    } else if constexpr (FMT == kQ5_0) {
+        const size_t o = (size_t)(j0 >> 5) * R + r;
+        k.v[0] = ld16(t.pa + o * 16);
+        k.v[1].x = ld4(t.pb + o * 4);
+        k.a = ld2(t.pd + o * 2);
+    } else if constexpr (FMT == kQ4_K) {
+        const int b = j0 >> 8, s = (j0 & 255) >> 5;
+        k.v[0] = ld16(t.pb + p16(b, 0, 1, R, r));
+        k.v[1] = ld16(t.pa + p16(b, (s >> 1) * 2, 8, R, r));
+        k.v[2] = ld16(t.pa + p16(b, (s >> 1) * 2 + 1, 8, R, r));
+    } else if constexpr (FMT == kQ6_K) {
+        const int b = j0 >> 8, off = j0 & 255, half = off >> 7, sub = (off & 127) >> 5;
+        const int cl = half * 4 + (sub & 1) * 2, ch = half * 2;
+        k.v[0] = ld16(t.pa + p16(b, cl, 8, R, r));
+        k.v[1] = ld16(t.pa + p16(b, cl + 1, 8, R, r));
+        k.v[2] = ld16(t.pb + p16(b, ch, 4, R, r));
+        k.v[3] = ld16(t.pb + p16(b, ch + 1, 4, R, r));
+        k.v[4] = ld16(t.pc + p16(b, 0, 1, R, r));
+        k.a = ld2(t.pd + ((size_t)b * R + r) * 2);
+    } else if constexpr (FMT == kF32) {
+#pragma unroll
+        for (int c = 0; c < 8; c++) k.v[c] = ld16(t.pa + p16(j0 >> 5, c, 8, R, r));
+    } else {  // F16
+#pragma unroll
+        for (int c = 0; c < 4; c++) k.v[c] = ld16(t.pa + p16(j0 >> 5, c, 4, R, r));
+    }
+}
+template <int FMT>
+__device__ __forceinline__ void dec32(const Raw32& k, int j0, float (&E)[32]) {
+    if constexpr (FMT == kQ8_0) {
+        const float d = h2f(k.a);
 #pragma unroll
         for (int i = 0; i < 16; i++) {
-            E[i] = (float)(int8_t)byte_of(v0, i) * d;
-            E[16 + i] = (float)(int8_t)byte_of(v1, i) * d;
+            E[i] = (float)(int8_t)byte_of(k.v[0], i) * d;
+            E[16 + i] = (float)(int8_t)byte_of(k.v[1], i) * d;
         }
-    } else if (t.type == kQ5_0) {
-        const int b = j0 >> 5;
-        const size_t o = (size_t)b * R + r;
-        const uint4 qs = ld16(t.pa + o * 16);
-        const uint32_t d4 = ld4(t.pb + o * 4);
-        const float d = h2f(ld2(t.pd + o * 2));
+    } else if constexpr (FMT == kQ5_0) {
+        const float d = h2f(k.a);
 #pragma unroll
-        for (int e = 0; e < 32; e++) E[e] = d * (float)(q5_code(qs, d4, e) - 16);
-    } else if (t.type == kQ4_K) {
-        const int b = j0 >> 8, s = (j0 & 255) >> 5;
-        const uint4 h = ld16(t.pb + p16(b, 0, 1, R, r));
-        const uint4 qa = ld16(t.pa + p16(b, (s >> 1) * 2, 8, R, r)), qb = ld16(t.pa + p16(b, (s >> 1) * 2 + 1, 8, R, r));
+        for (int e = 0; e < 32; e++) E[e] = d * (float)(q5_code(k.v[0], k.v[1].x, e) - 16);
+    } else if constexpr (FMT == kQ4_K) {
+        const int s = (j0 & 255) >> 5;
+        const uint4 h = k.v[0];
         const float d = h2f(h.x), dmin = h2f(h.x >> 16);
         int sc, m;
         q4k_scale_min(h, s, sc, m);
 #pragma unroll
         for (int i = 0; i < 32; i++) {
-            const uint32_t by = byte_of(i < 16 ? qa : qb, i & 15);
+            const uint32_t by = byte_of(i < 16 ? k.v[1] : k.v[2], i & 15);
             const int q4 = (s & 1) ? (int)(by >> 4) : (int)(by & 15u);
             E[i] = d * (float)sc * (float)q4 - dmin * (float)m;
         }
-    } else if (t.type == kQ6_K) {
-        const int b = j0 >> 8, off = j0 & 255, half = off >> 7, sub = (off & 127) >> 5;
-        const int cl = half * 4 + (sub & 1) * 2, ch = half * 2;
-        const uint4 l0 = ld16(t.pa + p16(b, cl, 8, R, r)), l1 = ld16(t.pa + p16(b, cl + 1, 8, R, r));
-        const uint4 h0 = ld16(t.pb + p16(b, ch, 4, R, r)), h1 = ld16(t.pb + p16(b, ch + 1, 4, R, r));
-        const uint4 scv = ld16(t.pc + p16(b, 0, 1, R, r));
-        const float d = h2f(ld2(t.pd + ((size_t)b * R + r) * 2));
+    } else if constexpr (FMT == kQ6_K) {
+        const int off = j0 & 255, half = off >> 7, sub = (off & 127) >> 5;
+        const float d = h2f(k.a);
 #pragma unroll
         for (int l = 0; l < 32; l++) {
-            const uint32_t qlb = byte_of(l < 16 ? l0 : l1, l & 15), qhb = byte_of(l < 16 ? h0 : h1, l & 15);
+            const uint32_t qlb = byte_of(l < 16 ? k.v[0] : k.v[1], l & 15), qhb = byte_of(l < 16 ? k.v[2] : k.v[3], l & 15);
             const uint32_t nib = (sub < 2) ? (qlb & 15u) : (qlb >> 4);
             const int q = (int)(nib | (((qhb >> (2 * sub)) & 3u) << 4)) - 32;
-            const int sc = (int)(int8_t)byte_of(scv, half * 8 + (l >> 4) + sub * 2);
+            const int sc = (int)(int8_t)byte_of(k.v[4], half * 8 + (l >> 4) + sub * 2);
             E[l] = d * (float)sc * (float)q;
         }
-    } else if (t.type == kF32) {
-        const int b = j0 >> 5;
+    } else if constexpr (FMT == kF32) {
 #pragma unroll
         for (int c = 0; c < 8; c++) {
-            const uint4 v = ld16(t.pa + p16(b, c, 8, R, r));
-            E[4 * c] = __uint_as_float(v.x);
-            E[4 * c + 1] = __uint_as_float(v.y);
-            E[4 * c + 2] = __uint_as_float(v.z);
-            E[4 * c + 3] = __uint_as_float(v.w);
+            E[4 * c] = __uint_as_float(k.v[c].x);
+            E[4 * c + 1] = __uint_as_float(k.v[c].y);
+            E[4 * c + 2] = __uint_as_float(k.v[c].z);
+            E[4 * c + 3] = __uint_as_float(k.v[c].w);
         }
     } else {  // F16
-        const int b = j0 >> 5;
 #pragma unroll
         for (int c = 0; c < 4; c++) {
-            const uint4 v = ld16(t.pa + p16(b, c, 4, R, r));
 #pragma unroll
-            for (int k = 0; k < 4; k++) {
-                const uint32_t w = dw_of(v, k);
-                E[8 * c + 2 * k] = h2f(w);
-                E[8 * c + 2 * k + 1] = h2f(w >> 16);
+            for (int i = 0; i < 4; i++) {
+                const uint32_t w = dw_of(k.v[c], i);
+                E[8 * c + 2 * i] = h2f(w);
+                E[8 * c + 2 * i + 1] = h2f(w >> 16);
             }
         }
+    }
+}
+template <int FMT>
+__device__ __forceinline__ void elems32_of(const TmqTensorDev& t, int r, int j0, float (&E)[32]) {
+    Raw32 k;
+    raw32<FMT>(t, r, j0, k);
+    dec32<FMT>(k, j0, E);
+}
+__device__ __forceinline__ void elems32(const TmqTensorDev& t, int r, int j0, float (&E)[32]) {
+    switch (t.type) {
+    case kQ8_0: elems32_of<kQ8_0>(t, r, j0, E); break;
+    case kQ5_0: elems32_of<kQ5_0>(t, r, j0, E); break;
+    case kQ4_K: elems32_of<kQ4_K>(t, r, j0, E); break;
+    case kQ6_K: elems32_of<kQ6_K>(t, r, j0, E); break;
+    case kF32: elems32_of<kF32>(t, r, j0, E); break;
+    default: elems32_of<kF16>(t, r, j0, E); break;
     }
 }
 
@@ -2106,6 +2147,92 @@ __global__ __launch_bounds__(64 * TMQ_WAVES) void f32_gemv_kernel(TmqWork w) {
         for (int i = 0; i < 32; i++) sum = sum + E[i] * __uint_as_float(xp[j0 + i]);
     }
     if (w.y && r < t.rows) store_y(w, r, sum);
+}
+
+// The same sums for few rows, where a lane that loads, decodes, multiplies
+// and adds its whole row is all latency.  Only the adds of a row depend on
+// each other, so wave 0 does nothing else: 16 rows a workgroup, its lane i
+// adds row i's products in column order from LDS while waves 1..3 make the
+// next kF32Cols columns' (lane 16 s + i: row i, the s-th 32 of the wave's 128
+// columns) and load the columns after those.  Bound by the adds and the
+// reads in front of them, 7.4 cycles a column (reads kept in flight behind
+// the adds, singly or in two sets of eight, were slower: 7.9-11 cycles).
+// A call: 4864 x 896 23.3 -> 6.2 us, 896 x 4864 122 -> 19.
+constexpr int kF32Rows = 16, kF32Prod = 3, kF32Cols = 128 * kF32Prod;
+constexpr int kF32Ld = kF32Cols + 4;  // (4: the 16 rows' float4 reads on different banks)
+template <int FMT>
+__global__ __launch_bounds__(64 * (1 + kF32Prod)) void f32_rows_kernel(TmqWork w) {
+    __shared__ __attribute__((aligned(16))) float prod[2][kF32Rows][kF32Ld];
+    __shared__ __attribute__((aligned(16))) float xs[kF32Prod][128];
+    const TmqTensorDev& t = w.t;
+    const int lane = threadIdx.x & 63, wave = wave_id();
+    const int row = lane & (kF32Rows - 1), r0 = blockIdx.x * kF32Rows;
+    const int n = t.cols, nbat = (n + kF32Cols - 1) / kF32Cols;
+    // batch k is made before barrier k and added after it, while batch k + 1
+    // goes to the other buffer (its batch k - 1 was added before barrier k)
+    auto barrier = [] { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
+    if (wave > 0) {
+        const int p = wave - 1, off = 128 * p + 32 * (lane >> 4);
+        struct Set {
+            Raw32 raw;
+            float x0, x1;
+        } A, B;
+        // (columns past the row's last block re-read it)
+        auto load = [&](Set& s, int k) {
+            const int j = kF32Cols * k + 128 * p + lane;
+            s.x0 = w.xf[min(j, n - 1)];
+            s.x1 = w.xf[min(j + 64, n - 1)];
+            raw32<FMT>(t, r0 + row, min(kF32Cols * k + off, n - 32), s.raw);
+        };
+        auto make = [&](const Set& s, int k) {
+            xs[p][lane] = s.x0;
+            xs[p][64 + lane] = s.x1;
+            float E[32];
+            dec32<FMT>(s.raw, min(kF32Cols * k + off, n - 32), E);
+            // (this wave's own x: its writes are done before its reads)
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            const float4* X = (const float4*)(xs[p] + 32 * (lane >> 4));
+            float4* d = (float4*)(prod[k & 1][row] + off);
+#pragma unroll
+            for (int i = 0; i < 8; i++) {
+                const float4 x = X[i];
+                d[i] = make_float4(E[4 * i] * x.x, E[4 * i + 1] * x.y, E[4 * i + 2] * x.z, E[4 * i + 3] * x.w);
+            }
+        };
+        // two register sets in turn, so that no copy waits on a load
+        load(A, 0);
+        for (int k = 0; k < nbat; k += 2) {
+            load(B, k + 1);
+            __builtin_amdgcn_sched_barrier(0);
+            make(A, k);
+            barrier();
+            if (k + 1 >= nbat) break;
+            load(A, k + 2);
+            __builtin_amdgcn_sched_barrier(0);
+            make(B, k + 1);
+            barrier();
+        }
+        return;
+    }
+    float sum = 0.0f;
+    for (int k = 0; k < nbat; k++) {
+        barrier();
+        const float4* d = (const float4*)prod[k & 1][row];
+        const int nq = min(kF32Cols, n - kF32Cols * k) / 32;
+        for (int q = 0; q < nq; q++) {
+            float4 v[8];
+#pragma unroll
+            for (int i = 0; i < 8; i++) v[i] = d[8 * q + i];
+#pragma unroll
+            for (int i = 0; i < 8; i++) {
+                sum += v[i].x;
+                sum += v[i].y;
+                sum += v[i].z;
+                sum += v[i].w;
+            }
+        }
+    }
+    if (w.y && lane < kF32Rows && r0 + row < t.rows) store_y(w, r0 + row, sum);
 }
 
 // ------------------------------------------------------------ engine GEMV
@@ -3829,8 +3956,24 @@ int tmq_launch_gemv(const TmqWork& w, hipStream_t s) {
             hipLaunchKernelGGL(i16_gemv_kernel, dim3(w.t.rows_pad / kI16Rows), dim3(64 * i16_waves(w.t.cols)),
                                i16_lds(w.t.cols), s, w);
         } else {
-            const int g = (w.t.rows_pad / 64 + TMQ_WAVES - 1) / TMQ_WAVES;
-            hipLaunchKernelGGL(f32_gemv_kernel, dim3(g), dim3(64 * TMQ_WAVES), 0, s, w);
+            // above this many rows a lane a row fills the chip (65000 x 896
+            // 30 us either way; 151936 x 896 35 us, 69 on f32_rows_kernel;
+            // 32768 x 896 31 against 17)
+            if (w.t.rows > 65536) {
+                const int g = (w.t.rows_pad / 64 + TMQ_WAVES - 1) / TMQ_WAVES;
+                hipLaunchKernelGGL(f32_gemv_kernel, dim3(g), dim3(64 * TMQ_WAVES), 0, s, w);
+                return (int)hipGetLastError();
+            }
+            const dim3 grid(w.t.rows_pad / kF32Rows), blk(64 * (1 + kF32Prod));
+            switch (w.t.type) {
+            case kQ8_0: hipLaunchKernelGGL(f32_rows_kernel<kQ8_0>, grid, blk, 0, s, w); break;
+            case kQ5_0: hipLaunchKernelGGL(f32_rows_kernel<kQ5_0>, grid, blk, 0, s, w); break;
+            case kQ4_K: hipLaunchKernelGGL(f32_rows_kernel<kQ4_K>, grid, blk, 0, s, w); break;
+            case kQ6_K: hipLaunchKernelGGL(f32_rows_kernel<kQ6_K>, grid, blk, 0, s, w); break;
+            case kF32: hipLaunchKernelGGL(f32_rows_kernel<kF32>, grid, blk, 0, s, w); break;
+            case kF16: hipLaunchKernelGGL(f32_rows_kernel<kF16>, grid, blk, 0, s, w); break;
+            default: return (int)hipErrorInvalidValue;
+            }
         }
         return (int)hipGetLastError();
     }
