@@ -51,7 +51,37 @@ def test_fp32_edges(ctx, oracle, qt, rows, cols):
     assert np.array_equal(bits(y), bits(oracle.matmul_fp32(qt, w, x, rows, cols)))
 
 
-@pytest.mark.parametrize("path", ["int16"])
+# the 16-row MFMA GEMVs: 1 and 3 blocks of a step's 4, 8 waves' worth (32) and
+# one step more, the widest; one and two super-blocks, more than 8 waves', the
+# bounds of the x registers (1024, 5120); rows 1, 16k, 16k + 1, and the first
+# row count past the rule
+@pytest.mark.parametrize("qt,rows,cols", [
+    (Q5_0, 1, 32), (Q5_0, 17, 96), (Q5_0, 48, 1024), (Q5_0, 65, 1056), (Q5_0, 16, 8192), (Q5_0, 16385, 96),
+    (Q4_K, 1, 256), (Q4_K, 33, 1024), (Q4_K, 64, 1280), (Q4_K, 15, 8192),
+    (Q6_K, 1, 256), (Q6_K, 31, 512), (Q6_K, 80, 5120), (Q6_K, 17, 5376), (Q6_K, 4097, 8192)])
+@pytest.mark.parametrize("force", [0, 1])
+def test_fpga_edges(ctx, oracle, monkeypatch, qt, rows, cols, force):
+    if force and rows > 100:
+        pytest.skip("the corrections' path is the same at every row count")
+    print(f"[single] fpga type={qt} {rows}x{cols} force={force}", flush=True)
+    if force:
+        monkeypatch.setenv("TMQ_IFIT_FORCE", "1")
+    w = synth.gen_weights(qt, rows, cols, 71 + rows)
+    x = synth.gen_x(cols, 72 + cols)
+    t = ctx.upload(qt, rows, cols, w)
+    try:
+        acc, xs = ctx.partials(t, x)
+        y = ctx.matmul(t, x)
+        z = ctx.matmul(t, np.zeros_like(x))
+    finally:
+        t.free()
+    assert xs == oracle.quantize_act(x)[1]
+    assert np.array_equal(bits(y), bits(oracle.matmul(qt, w, x, rows, cols)))
+    assert np.array_equal(bits(z), bits(oracle.matmul(qt, w, np.zeros_like(x), rows, cols)))
+    assert acc.shape == (rows,)
+
+
+@pytest.mark.parametrize("path", ["int16", "fpga"])
 def test_result_over_activation(ctx, oracle, path):
     """y written where x lies: every row still reads the whole x"""
     import torch
@@ -59,15 +89,19 @@ def test_result_over_activation(ctx, oracle, path):
     n = 896
     w = synth.gen_weights(Q5_0, n, n, 51)
     x = synth.gen_x(n, 52)
+    want = oracle.matmul_int16(Q5_0, w, x, n, n)[0] if path == "int16" else oracle.matmul(Q5_0, w, x, n, n)
     t = ctx.upload(Q5_0, n, n, w)
     try:
         for off in (0, 64, -64):
             buf = torch.zeros(n + 128, dtype=torch.float32, device="cuda")
             buf[64:64 + n] = torch.from_numpy(x)
             torch.cuda.synchronize()
-            ctx.gemv_dev_path(t, {"int16": tmq.PATH_INT16}[path], buf.data_ptr() + 256, buf.data_ptr() + 256 + 4 * off)
+            xp, yp = buf.data_ptr() + 256, buf.data_ptr() + 256 + 4 * off
+            if path == "int16":
+                ctx.gemv_dev_path(t, tmq.PATH_INT16, xp, yp)
+            else:
+                (ctx.gemv_dev if off else ctx.gemv_dev_noalloc)(t, xp, yp)
             ctx.sync()
-            y = buf[64 + off:64 + off + n].cpu().numpy()
-            assert np.array_equal(bits(y), bits(oracle.matmul_int16(Q5_0, w, x, n, n)[0])), off
+            assert np.array_equal(bits(buf[64 + off:64 + off + n].cpu().numpy()), bits(want)), off
     finally:
         t.free()

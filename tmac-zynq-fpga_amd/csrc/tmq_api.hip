@@ -433,17 +433,37 @@ TmqWork make_work(const tmq_tensor* t, const uint8_t* act, float* y, int64_t* ac
 
 // The activation a launch may read in every workgroup while others store
 // their results: x itself, or, where y or acc (acc_per int64 a row) lies over
-// it, a copy in the context's activation buffer (behind its x_scale).
-int own_x(tmq_ctx* ctx, const tmq_tensor* t, const float* x, const float* y, const int64_t* acc, size_t acc_per,
-          const float** out) {
+// it, a copy in the activation buffer `act` (behind its x_scale).
+int own_x(tmq_ctx* ctx, const tmq_tensor* t, uint8_t* act, const float* x, const float* y, const int64_t* acc,
+          size_t acc_per, const float** out) {
     const uintptr_t x0 = (uintptr_t)x, x1 = x0 + sizeof(float) * (size_t)t->dev.cols;
     auto over = [&](const void* p, size_t n) { return p && (uintptr_t)p < x1 && x0 < (uintptr_t)p + n; };
     *out = x;
     if (!over(y, sizeof(float) * (size_t)t->dev.rows) && !over(acc, sizeof(int64_t) * acc_per * (size_t)t->dev.rows))
         return 0;
-    float* c = (float*)((uint8_t*)ctx->act.p + 16);
+    float* c = (float*)(act + 16);
     HIP_TRY(hipMemcpyAsync(c, x, sizeof(float) * (size_t)t->dev.cols, hipMemcpyDeviceToDevice, ctx->stream));
     *out = c;
+    return 0;
+}
+
+// A tensor's own kernel on a device activation; `act` (tmq_act_bytes) gets
+// x_scale and, where the kernel reads one, the prepared activation.
+int gemv_fpga(tmq_ctx* ctx, const tmq_tensor* t, uint8_t* act, const float* x, float* y, int64_t* acc) {
+    TmqWork w = make_work(t, act, y, acc);
+    if (tmq_gemv_takes_x(t->dev)) {
+        const int rc = own_x(ctx, t, act, x, y, acc, t->dev.type == TMQ_TYPE_Q8_0 ? (t->dev.cols + 63) / 64 : 1, &w.xf);
+        if (rc) return rc;
+        w.xs_out = (float*)act;
+    } else {
+        TmqActJobs jobs{};
+        jobs.count = 1;
+        jobs.j[0].x = x;
+        jobs.j[0].act = act;
+        jobs.j[0].n = t->dev.cols;
+        LAUNCH_TRY(tmq_launch_act_prep(jobs, ctx->stream));
+    }
+    LAUNCH_TRY(tmq_launch_gemv(w, ctx->stream));
     return 0;
 }
 
@@ -626,6 +646,9 @@ int tmq_open(int device, tmq_ctx** out) {
         return tmq_fail(TMQ_ERR_HIP, "stream create: %s", hipGetErrorString(e));
     }
     int rc = scratch_init(device);
+    if (!rc)
+        if (const int pe = tmq_gemv_prepare())
+            rc = tmq_fail(TMQ_ERR_HIP, "GEMV set-up: %s", hipGetErrorString((hipError_t)pe));
     if (rc) {
         (void)hipStreamDestroy(c->stream);
         delete c;
@@ -737,16 +760,7 @@ int tmq_gemv_dev(tmq_ctx* ctx, const tmq_tensor* t, const float* x_dev, float* y
                         "matmul_fpga_int16 or the FP32 loop: tmq_gemv_dev_path)", type_name((uint32_t)t->dev.type));
     int rc = tmq_rt_set_device(ctx);
     if (!rc) rc = ctx->act.ensure(tmq_act_bytes(t->dev.cols));
-    if (rc) return rc;
-    TmqActJobs jobs{};
-    jobs.count = 1;
-    jobs.j[0].x = x_dev;
-    jobs.j[0].act = (uint8_t*)ctx->act.p;
-    jobs.j[0].n = t->dev.cols;
-    LAUNCH_TRY(tmq_launch_act_prep(jobs, ctx->stream));
-    TmqWork w = make_work(t, (const uint8_t*)ctx->act.p, y_dev, acc_dev);
-    LAUNCH_TRY(tmq_launch_gemv(w, ctx->stream));
-    return 0;
+    return rc ? rc : gemv_fpga(ctx, t, (uint8_t*)ctx->act.p, x_dev, y_dev, acc_dev);
 }
 
 int tmq_gemv_dev_noalloc(tmq_ctx* ctx, const tmq_tensor* t, const float* x_dev, float* y_dev, int64_t* acc_dev) {
@@ -760,15 +774,7 @@ int tmq_gemv_dev_noalloc(tmq_ctx* ctx, const tmq_tensor* t, const float* x_dev, 
     if (rc) return rc;
     uint8_t* act = (uint8_t*)scratch_of(ctx->device);
     if (!act) return tmq_fail(TMQ_ERR_HIP, "tmq_gemv_dev_noalloc: no scratch for device %d", ctx->device);
-    TmqActJobs jobs{};
-    jobs.count = 1;
-    jobs.j[0].x = x_dev;
-    jobs.j[0].act = act;
-    jobs.j[0].n = t->dev.cols;
-    LAUNCH_TRY(tmq_launch_act_prep(jobs, ctx->stream));
-    TmqWork w = make_work(t, act, y_dev, acc_dev);
-    LAUNCH_TRY(tmq_launch_gemv(w, ctx->stream));
-    return 0;
+    return gemv_fpga(ctx, t, act, x_dev, y_dev, acc_dev);
 }
 
 int tmq_matmul(tmq_ctx* ctx, const tmq_tensor* t, const float* x, float* y, int rows, int cols) {
@@ -882,7 +888,7 @@ int tmq_gemv_dev_path(tmq_ctx* ctx, const tmq_tensor* t, int path, const float* 
     if (rc) return rc;
     w = make_work(t, nullptr, y_dev, acc_dev);
     w.path = TMQ_WPATH_INT16;
-    rc = own_x(ctx, t, x_dev, y_dev, acc_dev, (size_t)((t->dev.cols + 63) / 64), &w.xf);
+    rc = own_x(ctx, t, (uint8_t*)ctx->act.p, x_dev, y_dev, acc_dev, (size_t)((t->dev.cols + 63) / 64), &w.xf);
     if (rc) return rc;
     w.xs_out = (float*)ctx->act.p;
     LAUNCH_TRY(tmq_launch_gemv(w, ctx->stream));

@@ -258,7 +258,14 @@ static inline int tmq_ifit_subs(int type) { return type == 6 ? 1 : type == 12 ? 
 #define TMQ_MFMA_MAX_COLS 8192
 int tmq_launch_rowstat(const TmqTensorDev& t, const float* aux_max_abs, float* row_inv,
                        float* row_scale, int* bad_flag, hipStream_t s);
+// A GEMV from a prepared activation (w.act), or, where w.xf is set instead
+// (INT16 and FP32 works, and FPGA works of a tensor that tmq_gemv_takes_x
+// says yes to), from the fp32 activation itself; x_scale goes to *w.xs_out
+// (not FP32).  With w.xf no result may lie over the activation.
 int tmq_launch_gemv(const TmqWork& w, hipStream_t s);
+bool tmq_gemv_takes_x(const TmqTensorDev& t);
+// before the first of them on a device (current): their kernels' LDS limits
+int tmq_gemv_prepare();
 // One workgroup of a chain launch: row group `group` of works[work] over
 // super-blocks [b0, b1) (b1 = 0: the whole row).  A K-quant MFMA group split
 // into `pieces` > 1 workgroups adds its int64 row sums into tail slot

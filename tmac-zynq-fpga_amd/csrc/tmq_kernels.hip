@@ -14,6 +14,8 @@
 // accumulates w*xh and w*xl pairs in int32 (|sum| < 2^28 per 32-weight
 // block), folded into int64 once per block.
 #include <hip/hip_runtime.h>
+
+#include <algorithm>
 #include <mutex>
 #include <set>
 
@@ -1180,18 +1182,30 @@ __device__ __forceinline__ tmq_v4i mfma16(tmq_v4i a, tmq_v4i b, tmq_v4i c) {
 // workgroup loads anyway), so that code around it sees a fixed number of
 // memory operations.  Returns the row's sum in wave 0 (after a workgroup
 // barrier; the other waves' values are meaningless).
-template <int NW, bool STATIC_PRIME = false, class Ready, class XQ>
+// RG16: group g is rows 16g .. 16g + 15 instead, lane 16q + n holding row n
+// and, of every four blocks, the q-th (K group q's A rows then hold that
+// block's activation), so that four times as many workgroups share the rows
+// and a wave's step covers four blocks.  [b0, b1) is the whole row; block
+// counts are in steps of four, whose surplus blocks re-read the last one
+// against zeros (the caller pads xa and xsl with them).  Every lane of wave
+// 0 returns its row's sum.
+template <int NW, bool STATIC_PRIME = false, bool RG16 = false, class Ready, class XQ>
 __device__ __forceinline__ int64_t mfma_q5_rows(const TmqTensorDev& t, int g, int b0, int b1, const uint8_t* xa,
                                                 const int32_t* xsl, uint8_t* ring0, int64_t* part, int clo, int chi,
                                                 Ready&& ready, XQ&& xq) {
-    constexpr int D = TMQ_MFMA_DEPTH;
+    constexpr int D = TMQ_MFMA_DEPTH, RG = RG16 ? 16 : 64;
     const int nb = t.nb;
     const int lane = threadIdx.x & 63, wave = wave_id();
-    const int r = g * 64 + lane;
+    const int r = g * RG + (lane & (RG - 1)), q4 = RG16 ? lane >> 4 : 0;
+    if (RG16) {
+        b0 = 0;
+        b1 = (nb + 3) / 4;
+    }
     const int nbw = max(0, (b1 - b0 - wave + NW - 1) / NW);  // this wave's blocks (wave-uniform)
     // corrections of the group (uniform), fetched first
     const bool corr = t.corr_off && chi > clo;
-    const int c0 = corr ? t.corr_off[g] : 0, c1 = corr ? t.corr_off[g + 1] : 0;
+    const int cg = RG16 ? g >> 2 : g;
+    const int c0 = corr ? t.corr_off[cg] : 0, c1 = corr ? t.corr_off[cg + 1] : 0;
     const float inv = t.row_inv[r], ri256 = inv * 256.0f;
     int64_t* fix = part + NW * 64;
 
@@ -1213,8 +1227,17 @@ __device__ __forceinline__ int64_t mfma_q5_rows(const TmqTensorDev& t, int g, in
         // last block, or the range's first when it has none)
         const int blk = __builtin_amdgcn_readfirstlane(
             i < nbw ? b0 + wave + NW * i : nbw > 0 ? b0 + wave + NW * (nbw - 1) : min(b0, nb - 1));
-        const int ob = blk * (int)R + g * 64;
         uint8_t* st = ring + slot * kMfmaStage;
+        if constexpr (RG16) {
+            const int o = (min(4 * blk + q4, nb - 1)) * (int)R + r;
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rsa, (lds_u8*)st, 16, 16 * o, 0, 0, TMQ_CPOL_NT);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rsb, (lds_u8*)(st + 1024), 4, 4 * o, 0, 0, TMQ_CPOL_NT);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rsd, (lds_u8*)(st + 1280), 2, 2 * o, 0, 0, TMQ_CPOL_NT);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rsi, (lds_u8*)(st + 1536), 4, 4 * (blk * (int)R + r), 0, 0,
+                                                     TMQ_CPOL_NT);
+            return;
+        }
+        const int ob = blk * (int)R + g * 64;
         __builtin_amdgcn_raw_ptr_buffer_load_lds(rsa, (lds_u8*)st, 16, la16, 16 * ob, 0, TMQ_CPOL_NT);
         __builtin_amdgcn_raw_ptr_buffer_load_lds(rsb, (lds_u8*)(st + 1024), 4, la4, 4 * ob, 0, TMQ_CPOL_NT);
         __builtin_amdgcn_raw_ptr_buffer_load_lds(rsd, (lds_u8*)(st + 1280), 2, la2, 2 * ob, 0, TMQ_CPOL_NT);
@@ -1240,9 +1263,9 @@ __device__ __forceinline__ int64_t mfma_q5_rows(const TmqTensorDev& t, int g, in
     {
         const int q = lane >> 4, m = lane & 15, dg = m & 3;
         const bool own = (m >> 2) == q;
-        const uint32_t zero = (uint32_t)nb * 64u;
-        const uint32_t abase = own && dg < 2 ? (uint32_t)(dg * 16) : own && dg == 2 ? zero + kMfmaConst / 2 : zero;
-        astride = own && dg < 2 ? 64u : 0u;
+        const uint32_t zero = (uint32_t)(RG16 ? (nb + 3) & ~3 : nb) * 64u;
+        const uint32_t abase = own && dg < 2 ? (uint32_t)(64 * q4 + dg * 16) : own && dg == 2 ? zero + kMfmaConst / 2 : zero;
+        astride = own && dg < 2 ? (RG16 ? 256u : 64u) : 0u;
         ap0 = (const lds_u8*)(xa + abase);
     }
 
@@ -1272,10 +1295,10 @@ __device__ __forceinline__ int64_t mfma_q5_rows(const TmqTensorDev& t, int g, in
         }
         k.qh = *(lu32c*)(st + 1024 + lane * 4);
         k.d = *(lu16*)(st + 1280 + lane * 4);
-        k.e = *(lu8*)(st + 1536 + lane * 4 + (b & 3));
+        k.e = *(lu8*)(st + 1536 + lane * 4 + (RG16 ? q4 : b & 3));
         const lds_u8* xp0 = ap0 + (uint32_t)b * astride;
         const tmq_v4i A0 = *(lv4i*)xp0, A1 = *(lv4i*)(xp0 + 32);
-        const int xsv = *(li32*)(xsl + b);
+        const int xsv = *(li32*)(xsl + (RG16 ? 4 * b + q4 : b));
         // the stage's reads are in registers before its refill overwrites it
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         if (FULL || i + D < nbw) issue(i + D, slot);
@@ -1321,17 +1344,22 @@ __device__ __forceinline__ int64_t mfma_q5_rows(const TmqTensorDev& t, int g, in
             const uint4 e = t.corr[c];
             // (a correction's elements lie in one block or sub-block)
             if ((int)e.y < clo || (int)e.y >= chi) continue;
+            if (RG16 && (int)e.x >> 4 != g) continue;
             int64_t s = 0;
             for (uint32_t m = e.z; m; m &= m - 1) s += xq((int)e.y + __builtin_ctz(m));
-            atomicAdd((unsigned long long*)&fix[(int)e.x - g * 64], (unsigned long long)((int64_t)(int32_t)e.w * s));
+            atomicAdd((unsigned long long*)&fix[(int)e.x - g * RG], (unsigned long long)((int64_t)(int32_t)e.w * s));
         }
         __syncthreads();
     }
     int64_t tot = 0;
     if (wave == 0) {
-        tot = fix[lane];
+        tot = RG16 && lane >= RG ? 0 : fix[lane];
 #pragma unroll
         for (int i = 0; i < NW; i++) tot += part[i * 64 + lane];
+        if constexpr (RG16) {  // the row's four lanes
+            tot += __shfl_xor(tot, 16);
+            tot += __shfl_xor(tot, 32);
+        }
     }
     return tot;
 }
@@ -1431,27 +1459,30 @@ template <int FMT> __host__ __device__ constexpr int kq_lds_bytes(int nbx) {
 // mfma_q5_rows (xs16l: Q6_K's 16-element sums; part (NW + 1) * 64 int64;
 // ring NW * D stages; xa's constant runs kKqConst bytes at xa + 64 * 8nb)
 // and the same ready / corr / xq contract.  Returns the rows' sums in wave 0.
-template <int FMT, bool STATIC_PRIME = false, class Ready, class XQ>
+// RG16 (see mfma_q5_rows): lane 16q + n holds row n and quarter q of the
+// wave's super-blocks w, w + NWV, ...
+template <int FMT, bool STATIC_PRIME = false, bool RG16 = false, int NWV = kKqWaves, class Ready, class XQ>
 __device__ __forceinline__ int64_t mfma_kq_rows(const TmqTensorDev& t, int g, int b0, int b1, const uint8_t* xa,
                                                 const int32_t* xsl, const int32_t* xs16l, uint8_t* ring0,
                                                 int64_t* part, int clo, int chi, Ready&& ready, XQ&& xq) {
-    constexpr int NW = kKqWaves, D = TMQ_MFMA_DEPTH, ST = kq_stage<FMT>(), ND = kq_ndma<FMT>();
+    constexpr int NW = NWV, D = TMQ_MFMA_DEPTH, ST = kq_stage<FMT>(), ND = kq_ndma<FMT>(), RG = RG16 ? 16 : 64;
     constexpr int NS = FMT == kQ4_K ? 2 : 4;  // sub-blocks per quarter
     const int nb = t.nb, nbx = nb * 8;
     const int lane = threadIdx.x & 63, wave = wave_id();
-    const int r = g * 64 + lane;
+    const int r = g * RG + (lane & (RG - 1)), q4 = lane >> 4;
     // quarter u = 4b + q of the row; wave w takes quarters u0 + w + NW*i:
     // quarter w of each super-block of the range (NW = 4 = quarters per
     // super-block), b1 - b0 >= 1 of them
     const int u0 = 4 * b0;
-    const int nuw = b1 - b0;
+    const int nuw = RG16 ? max(0, (b1 - b0 - wave + NW - 1) / NW) : b1 - b0;
     const bool corr = t.corr_off && chi > clo;
-    const int c0 = corr ? t.corr_off[g] : 0, c1 = corr ? t.corr_off[g + 1] : 0;
+    const int cg = RG16 ? g >> 2 : g;
+    const int c0 = corr ? t.corr_off[cg] : 0, c1 = corr ? t.corr_off[cg + 1] : 0;
     const float inv = t.row_inv[r], ri256 = inv * 256.0f;
     int64_t* fix = part + NW * 64;
 
     uint8_t* ring = ring0 + wave * D * ST;
-    const int R = t.rows_pad, g64 = g * 64;
+    const int R = t.rows_pad, g64 = g * RG;
     // planes (the host keeps each below 2^31 bytes)
     const uint32_t pb = (uint32_t)R * (uint32_t)nb;  // (row, block) pairs
     const __amdgpu_buffer_rsrc_t rsa = buf_rsrc(t.pa, 128 * pb), rsi = buf_rsrc(t.pi, (FMT == kQ4_K ? 8 : 16) * pb);
@@ -1464,11 +1495,35 @@ __device__ __forceinline__ int64_t mfma_kq_rows(const TmqTensorDev& t, int g, in
     auto issue = [&](int i, int slot) {
         // (i < nuw, but for a static prime's surplus stages: the last
         // quarter, or the row's first super-block's when the range is empty)
+        uint8_t* st = ring + slot * ST;
+        if constexpr (RG16) {
+            const int b = __builtin_amdgcn_readfirstlane(
+                b0 + (i < nuw ? wave + NW * i : nuw > 0 ? wave + NW * (nuw - 1) : 0));
+            if constexpr (FMT == kQ4_K) {
+                const int o = (b * 8 + 2 * q4) * R + r;
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(rsa, (lds_u8*)st, 16, o * 16, 0, 0, TMQ_CPOL_NT);
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(rsa, (lds_u8*)(st + 1024), 16, (o + R) * 16, 0, 0, TMQ_CPOL_NT);
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(rsb, (lds_u8*)(st + 2048), 16, (b * R + r) * 16, 0, 0, 0);
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(rsi, (lds_u8*)(st + 3072), 2, ((b * 4 + q4) * R + r) * 2, 0, 0,
+                                                         TMQ_CPOL_NT);
+            } else {
+                const int o = (b * 12 + 3 * q4) * R + r;
+#pragma unroll
+                for (int k = 0; k < 3; k++)
+                    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsq, (lds_u8*)(st + 1024 * k), 16, (o + k * R) * 16, 0, 0,
+                                                             TMQ_CPOL_NT);
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(rsq, (lds_u8*)(st + 3072), 4, ((b * 4 + q4) * R + r) * 4,
+                                                         (int)(192 * pb), 0, TMQ_CPOL_NT);
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(rsd, (lds_u8*)(st + 3328), 2, (b * R + r) * 2, 0, 0, 0);
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(rsi, (lds_u8*)(st + 3584), 4, ((b * 4 + q4) * R + r) * 4, 0, 0,
+                                                         TMQ_CPOL_NT);
+            }
+            return;
+        }
         const int u = __builtin_amdgcn_readfirstlane(i < nuw ? u0 + wave + NW * i
                                                      : nuw > 0 ? u0 + wave + NW * (nuw - 1)
                                                                : 4 * min(b0, nb - 1) + wave);
         const int b = u >> 2, q = u & 3;
-        uint8_t* st = ring + slot * ST;
         if constexpr (FMT == kQ4_K) {
             __builtin_amdgcn_raw_ptr_buffer_load_lds(rsa, (lds_u8*)st, 16, l16, ((b * 8 + 2 * q) * R + g64) * 16, 0,
                                                      TMQ_CPOL_NT);
@@ -1534,11 +1589,12 @@ __device__ __forceinline__ int64_t mfma_kq_rows(const TmqTensorDev& t, int g, in
     //           m_k = (scales[8 + s'] >> 4) | (scales[4 + s'] >> 6) << 4
     // gathered by v_perm as the bytes (sc_0, sc_1, m_0, m_1) of one dword:
     // bytes s0, s0 + 1 of a header dword and of the next, s0 = 2 * (q & 1)
-    static_assert(NW == 4, "the quarter of a wave is wave & 3");
-    const int qw = wave & 3;
+    // (RG16: a lane's own quarter, both cases formed)
+    static_assert(NW == 4 || RG16, "the quarter of a wave is wave & 3");
+    const int qw = RG16 ? q4 : wave & 3;
     const uint32_t hs0 = 2u * (uint32_t)(qw & 1);
-    const uint32_t hsel = (uint32_t)__builtin_amdgcn_readfirstlane(
-        (int)(hs0 | (hs0 + 1) << 8 | (hs0 + 4) << 16 | (hs0 + 5) << 24));
+    uint32_t hsel = hs0 | (hs0 + 1) << 8 | (hs0 + 4) << 16 | (hs0 + 5) << 24;
+    if (!RG16) hsel = (uint32_t)__builtin_amdgcn_readfirstlane((int)hsel);
     // the loop, compiled per header case (q < 2 or not; Q6_K: one case)
     auto run = [&](auto lo2c) {
         constexpr bool LO2 = decltype(lo2c)::value;
@@ -1550,7 +1606,7 @@ __device__ __forceinline__ int64_t mfma_kq_rows(const TmqTensorDev& t, int g, in
                 wait_vm<ND * (D - 1)>();
             else
                 wait_vm_k<ND, D - 1>(min(D - 1, nuw - 1 - i));
-            const int u = u0 + wave + NW * i, b = u >> 2, q = u & 3;
+            const int u = u0 + wave + NW * i, b = RG16 ? b0 + wave + NW * i : u >> 2, q = RG16 ? q4 : u & 3;
             const uint8_t* st = ring + slot * ST;
             IFit f[NS];
             tmq_v4i UA[NS][2], TA[NS][2], AA[NS][2];
@@ -1572,7 +1628,10 @@ __device__ __forceinline__ int64_t mfma_kq_rows(const TmqTensorDev& t, int g, in
                 const uint32_t hx = (uint32_t)hv.x, hy = (uint32_t)hv.y, hz = (uint32_t)hv.z, hw = (uint32_t)hv.w;
                 const float dri = h2f(hx) * ri256, mri = h2f(hx >> 16) * ri256;
                 uint32_t scm;
-                if constexpr (LO2)
+                if constexpr (RG16) {
+                    const uint32_t p1 = __builtin_amdgcn_perm(hz, hy, hsel), p2 = __builtin_amdgcn_perm(hw >> 4, hw, hsel);
+                    scm = qw < 2 ? p1 & 0x3f3f3f3fu : (p2 & 0x0f0f0f0fu) | ((p1 >> 2) & 0x30303030u);
+                } else if constexpr (LO2)
                     scm = __builtin_amdgcn_perm(hz, hy, hsel) & 0x3f3f3f3fu;
                 else
                     scm = (__builtin_amdgcn_perm(hw >> 4, hw, hsel) & 0x0f0f0f0fu) |
@@ -1666,7 +1725,7 @@ __device__ __forceinline__ int64_t mfma_kq_rows(const TmqTensorDev& t, int g, in
         for (int i = 0; i < 2 * D - 1; i++)
             if (ib + i < nuw) step(ib + i, i % D, BoolC<false>{});
     };
-    if constexpr (FMT == kQ4_K) {
+    if constexpr (FMT == kQ4_K && !RG16) {
         if (qw < 2)
             run(BoolC<true>{});
         else
@@ -1689,17 +1748,22 @@ __device__ __forceinline__ int64_t mfma_kq_rows(const TmqTensorDev& t, int g, in
             const uint4 e = t.corr[c];
             // (a correction's elements lie in one block or sub-block)
             if ((int)e.y < clo || (int)e.y >= chi) continue;
+            if (RG16 && (int)e.x >> 4 != g) continue;
             int64_t s = 0;
             for (uint32_t m = e.z; m; m &= m - 1) s += xq((int)e.y + __builtin_ctz(m));
-            atomicAdd((unsigned long long*)&fix[(int)e.x - g * 64], (unsigned long long)((int64_t)(int32_t)e.w * s));
+            atomicAdd((unsigned long long*)&fix[(int)e.x - g * RG], (unsigned long long)((int64_t)(int32_t)e.w * s));
         }
         __syncthreads();
     }
     int64_t tot = 0;
     if (wave == 0) {
-        tot = fix[lane];
+        tot = RG16 && lane >= RG ? 0 : fix[lane];
 #pragma unroll
         for (int i = 0; i < NW; i++) tot += part[i * 64 + lane];
+        if constexpr (RG16) {  // the row's four lanes
+            tot += __shfl_xor(tot, 16);
+            tot += __shfl_xor(tot, 32);
+        }
     }
     return tot;
 }
@@ -1824,6 +1888,113 @@ __global__ __launch_bounds__(64 * gemv_waves(FMT), FMT == kQ5_0M ? 8 : 1) void c
     const TmqWork* __restrict__ works, const TmqGroupRef* __restrict__ groups, uint64_t* tail) {
     const TmqGroupRef ref = groups[blockIdx.x];
     run_group<FMT, CLAMP>(works[ref.work], ref.group, ref.b0, ref.b1, ref.slot, ref.pieces, tail);
+}
+
+// -------------------------------------------------- single-launch GEMVs
+// x_scale and the MFMA operand bytes of x[0, n) (the layout act_prep_kernel
+// writes), made by the workgroup in LDS: bytes xa, sums over 32 (xsl) and 16
+// (xs16l, unless null) elements, nbx blocks of 32 (those past n zero) and
+// the constant runs of CB bytes behind them.  KX elements a thread, n <= KX *
+// 64 NW; prime() runs behind the loads of x, so that the weights it asks for
+// do not hold them up, and issues a fixed number of memory operations.
+template <int NW, int KX, int CB, class Prime>
+__device__ __forceinline__ float quant_lds(const float* __restrict__ x, int n, int nbx, uint8_t* xa, int32_t* xsl,
+                                           int32_t* xs16l, Prime&& prime) {
+    __shared__ float red[NW];
+    constexpr int NT = 64 * NW;
+    const int tid = threadIdx.x, lane = tid & 63, wave = wave_id();
+    auto barrier = [] { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
+    float v[KX];
+#pragma unroll
+    for (int k = 0; k < KX; k++) v[k] = x[min(tid + NT * k, n - 1)];
+    __builtin_amdgcn_sched_barrier(0);
+    prime();
+    __builtin_amdgcn_sched_barrier(0);
+    if (tid < CB / 16) {
+        const uint32_t c = tid < CB / 32 ? 0u : 0x01010101u;
+        *(uint4*)(xa + nbx * 64 + tid * 16) = make_uint4(c, c, c, c);
+    }
+    float m = 0.0f;
+#pragma unroll
+    for (int k = 0; k < KX; k++) m = fmaxf(m, fabsf(v[k]));
+    m = tmq_wave_max(m);
+    if (lane == 0) red[wave] = m;
+    barrier();
+    float mm = red[0];
+#pragma unroll
+    for (int i = 1; i < NW; i++) mm = fmaxf(mm, red[i]);
+    const float xs = (mm < 1e-10f) ? 1.0f : mm / 32767.0f;
+#pragma unroll
+    for (int k = 0; k < KX; k++) {
+        const int j = tid + NT * k;
+        if (NT * k >= 32 * nbx) break;  // (uniform)
+        const int q = j < n ? (int)(int16_t)roundf(v[k] / xs) : 0;
+        // 16 lanes hold 16 consecutive elements
+        const int s16 = tmq_row_sum(q), s32 = s16 + __shfl_xor(s16, 16);
+        if (j < 32 * nbx) {
+            uint8_t* d = xa + 64 * (j >> 5) + 32 * ((j >> 4) & 1) + (j & 15);
+            d[0] = (uint8_t)(q >> 8);
+            d[16] = (uint8_t)((q & 255) ^ 0x80);
+            if (xs16l && (j & 15) == 0) xs16l[j >> 4] = s16;
+            if ((j & 31) == 0) xsl[j >> 5] = s32;
+        }
+    }
+    barrier();
+    return xs;
+}
+// element col of a quantised x from those bytes
+__device__ __forceinline__ int32_t quant_elem(const uint8_t* xa, int col) {
+    const uint8_t* d = xa + 64 * (col >> 5) + 32 * ((col >> 4) & 1) + (col & 15);
+    return (int)(int8_t)d[0] * 256 + (int)(d[16] ^ 0x80);
+}
+
+// One GEMV of an MFMA format without a launch in front: 16 rows a workgroup
+// (mfma_*_rows<RG16>), 8 waves over the row's blocks, the activation
+// quantised by every workgroup.  x is w.xf; x_scale is left in *w.xs_out.
+// A small GEMV is latency: two launches, and in the second one wave a
+// quarter of the 64 rows' blocks one after another (896 x 4864: 14
+// workgroups).  A call: Q6_K 896 x 4864 21.7 -> 7.9 us, Q4_K 18.8 -> 6.8,
+// Q5_0 4864 x 896 9.5 -> 5.4, 128 x 896 9.3 -> 4.0.
+constexpr int kOneWaves = 8;
+__host__ __device__ constexpr int one_nbx(int cols) { return ((cols + 31) / 32 + 3) & ~3; }
+template <int FMT> __host__ __device__ constexpr int one_ring() {
+    return kOneWaves * TMQ_MFMA_DEPTH * (FMT == kQ5_0M ? kMfmaStage : kq_stage<FMT == kQ4_KM ? kQ4_K : kQ6_K>());
+}
+template <int FMT> __host__ __device__ constexpr int one_xs_off(int nbx) {
+    return one_ring<FMT>() + nbx * 64 + (FMT == kQ5_0M ? kMfmaConst : kKqConst);
+}
+template <int FMT> __host__ __device__ constexpr int one_part_off(int nbx) {
+    return one_xs_off<FMT>(nbx) + nbx * 4 + (FMT == kQ6_KM ? nbx * 8 : 0);
+}
+template <int FMT> __host__ __device__ constexpr int one_lds(int nbx) { return one_part_off<FMT>(nbx) + (kOneWaves + 1) * 64 * 8; }
+template <int FMT, int KX>
+__global__ __launch_bounds__(64 * kOneWaves) void one_kernel(TmqWork w) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t mfma_lds[];
+    tmq_warm_kernargs<sizeof(TmqWork)>();
+    const TmqTensorDev& t = w.t;
+    const int g = blockIdx.x, lane = threadIdx.x & 63, n = t.cols, nbx = one_nbx(n);
+    uint8_t* xa = mfma_lds + one_ring<FMT>();
+    int32_t* xsl = (int32_t*)(mfma_lds + one_xs_off<FMT>(nbx));
+    int32_t* xs16l = FMT == kQ6_KM ? xsl + nbx : nullptr;
+    int64_t* part = (int64_t*)(mfma_lds + one_part_off<FMT>(nbx));
+    const int r = g * 16 + (lane & 15);
+    const float inv = t.row_inv[r];
+    float xsc = 0.0f;
+    auto ready = [&](auto&& prime, int) {
+        xsc = quant_lds<kOneWaves, KX, FMT == kQ5_0M ? kMfmaConst : kKqConst>(w.xf, n, nbx, xa, xsl, xs16l, prime);
+    };
+    auto xq = [&](int col) { return quant_elem(xa, col); };
+    int64_t tot;
+    if constexpr (FMT == kQ5_0M)
+        tot = mfma_q5_rows<kOneWaves, true, true>(t, g, 0, 0, xa, xsl, mfma_lds, part, 0, n, ready, xq);
+    else
+        tot = mfma_kq_rows<FMT == kQ4_KM ? kQ4_K : kQ6_K, true, true, kOneWaves>(t, g, 0, t.nb, xa, xsl, xs16l, mfma_lds,
+                                                                                 part, 0, n, ready, xq);
+    if (g == 0 && threadIdx.x == 0) *w.xs_out = xsc;
+    if (threadIdx.x < 16 && r < t.rows) {
+        if (w.acc) w.acc[r] = tot;
+        if (w.y) store_y(w, r, (float)(((double)tot * (double)xsc) / (double)inv));
+    }
 }
 
 // ------------------------------------------------- INT16 and FP32 paths
@@ -3946,6 +4117,28 @@ static void* kernel_for(int type, int clamp) {
 }
 template <int F, bool C> struct GemvK { static auto fn() { return gemv_kernel<F, C>; } };
 template <int F, bool C> struct ChainK { static auto fn() { return chain_kernel<F, C>; } };
+// the single-launch GEMVs' dynamic LDS limit, on the current device
+int tmq_gemv_prepare() {
+    const void* fns[] = {(const void*)one_kernel<kQ4_KM, 2>,  (const void*)one_kernel<kQ4_KM, 10>,
+                         (const void*)one_kernel<kQ4_KM, 16>, (const void*)one_kernel<kQ6_KM, 2>,
+                         (const void*)one_kernel<kQ6_KM, 10>, (const void*)one_kernel<kQ6_KM, 16>};
+    const int lds = std::max(one_lds<kQ4_KM>(one_nbx(TMQ_MFMA_MAX_COLS)), one_lds<kQ6_KM>(one_nbx(TMQ_MFMA_MAX_COLS)));
+    for (const void* f : fns) {
+        const hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+        if (e != hipSuccess) return (int)e;
+    }
+    return 0;
+}
+// One launch of 16-row workgroups up to where 64-row groups fill the chip:
+// the time grows with the weights (0.35 ns a row of 896 Q5_0, 0.62 of 1024
+// and 2.5 of 4096 Q6_K columns) where the two launches' is flat (10 us at
+// 896 columns, 12 at 1024, 20 at 4096, 32 at 8192).
+// Q5_0 16000 x 896 8.5 against 10.0 us, 65000 x 896 25.6 against 14.2;
+// Q6_K 20000 x 1024 14.7 against 12.1, 5000 x 4096 11.8 against 19.6.
+bool tmq_gemv_takes_x(const TmqTensorDev& t) {
+    const int f = tmq_kernel_fmt(t);
+    return (f == kQ5_0M || f == kQ4_KM || f == kQ6_KM) && t.rows <= 16384 && (int64_t)t.rows * t.cols <= 1 << 25;
+}
 int tmq_launch_gemv(const TmqWork& w, hipStream_t s) {
     if (w.ngroups <= 0) return 0;
     if (w.path != TMQ_WPATH_FPGA) {
@@ -3978,6 +4171,23 @@ int tmq_launch_gemv(const TmqWork& w, hipStream_t s) {
         return (int)hipGetLastError();
     }
     const int fmt = tmq_kernel_fmt(w.t);
+    if (w.xf) {
+        const int nbx = one_nbx(w.t.cols), kx = (w.t.cols + 64 * kOneWaves - 1) / (64 * kOneWaves);
+        const dim3 grid(w.t.rows_pad / 16), blk(64 * kOneWaves);
+        if (fmt == kQ5_0M) {
+            if (kx <= 2) hipLaunchKernelGGL((one_kernel<kQ5_0M, 2>), grid, blk, one_lds<kQ5_0M>(nbx), s, w);
+            else hipLaunchKernelGGL((one_kernel<kQ5_0M, 16>), grid, blk, one_lds<kQ5_0M>(nbx), s, w);
+        } else if (fmt == kQ4_KM) {
+            if (kx <= 2) hipLaunchKernelGGL((one_kernel<kQ4_KM, 2>), grid, blk, one_lds<kQ4_KM>(nbx), s, w);
+            else if (kx <= 10) hipLaunchKernelGGL((one_kernel<kQ4_KM, 10>), grid, blk, one_lds<kQ4_KM>(nbx), s, w);
+            else hipLaunchKernelGGL((one_kernel<kQ4_KM, 16>), grid, blk, one_lds<kQ4_KM>(nbx), s, w);
+        } else {
+            if (kx <= 2) hipLaunchKernelGGL((one_kernel<kQ6_KM, 2>), grid, blk, one_lds<kQ6_KM>(nbx), s, w);
+            else if (kx <= 10) hipLaunchKernelGGL((one_kernel<kQ6_KM, 10>), grid, blk, one_lds<kQ6_KM>(nbx), s, w);
+            else hipLaunchKernelGGL((one_kernel<kQ6_KM, 16>), grid, blk, one_lds<kQ6_KM>(nbx), s, w);
+        }
+        return (int)hipGetLastError();
+    }
     void* k = kernel_for<GemvK>(fmt, w.t.clamp);
     if (!k) return (int)hipErrorInvalidValue;
     TmqWork arg = w;
