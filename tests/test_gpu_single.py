@@ -105,3 +105,82 @@ def test_result_over_activation(ctx, oracle, path):
             assert np.array_equal(bits(buf[64 + off:64 + off + n].cpu().numpy()), bits(want)), off
     finally:
         t.free()
+
+
+def chain_of(ctx, torch, shapes, share=None):
+    """(chain, xs, x host, y, weights) of (type, rows, cols, activation) rows"""
+    import tmq
+    per = {Q5_0: 8, Q8_0: 64, Q4_K: 56, Q6_K: 32}
+    xh = {a: synth.gen_x(c, 90 + a) for _, _, c, a in shapes}
+    xs = {a: torch.from_numpy(x).cuda() for a, x in xh.items()}
+    ys = [torch.zeros(r, dtype=torch.float32, device="cuda") for _, r, _, _ in shapes]
+    if share:  # y of one descriptor over x of another
+        ys[share[0]] = xs[share[1]]
+    ws, descs, ts = [], [], []
+    for i, (qt, r, c, a) in enumerate(shapes):
+        w = synth.gen_weights(qt, r, c, 80 + i)
+        t = ctx.upload(qt, r, c, w)
+        p = max(k for k in range(1, per[qt] + 1) if r % k == 0)
+        cg = c // 256 if qt in (Q4_K, Q6_K) else 1
+        descs.append((t, xs[a].data_ptr(), ys[i].data_ptr(), None, r // p * cg, p, cg))
+        ws.append(w)
+        ts.append(t)
+    torch.cuda.synchronize()
+    return tmq.Chain(ctx, descs), xs, xh, ys, ws
+
+
+# every decoder of the one-launch chain with a ragged last workgroup: 16- and
+# 64-row Q5_0, wide Q5_0, Q8_0 of one half tile and of 8 waves' tiles and one
+# more, both K-quants at both register bounds
+CHAIN = [(Q5_0, 2050, 896, 0), (Q5_0, 17, 896, 0), (Q5_0, 33, 2048, 1), (Q8_0, 65, 96, 2), (Q8_0, 70, 544, 3),
+         (Q4_K, 9, 256, 4), (Q6_K, 18, 4864, 5), (Q4_K, 17, 5376, 6), (Q6_K, 31, 256, 4)]
+
+
+def test_chain_one_launch(ctx, oracle):
+    import torch
+    ch, xs, xh, ys, ws = chain_of(ctx, torch, CHAIN)
+    want = [oracle.matmul(qt, w, xh[a], r, c) for (qt, r, c, a), w in zip(CHAIN, ws)]
+    for rep in range(3):
+        for y in ys:
+            y.zero_()
+        torch.cuda.synchronize()
+        # the third time from the activations the last run prepared
+        (ch.launch if rep == 2 else ch.run)()
+        ctx.sync()
+        for (qt, r, c, a), y, e in zip(CHAIN, ys, want):
+            assert np.array_equal(bits(y.cpu().numpy()), bits(e)), (rep, qt, r, c)
+        if rep == 1:
+            for x in xs.values():
+                x.zero_()
+            torch.cuda.synchronize()
+    ch.free()
+
+
+def test_chain_result_over_activation(ctx, oracle):
+    """every activation is quantised before any result is stored"""
+    import torch
+    shapes = [(Q5_0, 896, 896, 0), (Q8_0, 100, 896, 1), (Q6_K, 20, 512, 2)]
+    ch, xs, xh, ys, ws = chain_of(ctx, torch, shapes, share=(0, 1))
+    ch.run()
+    ctx.sync()
+    for (qt, r, c, a), y, w in zip(shapes, ys, ws):
+        assert np.array_equal(bits(y.cpu().numpy()), bits(oracle.matmul(qt, w, xh[a], r, c))), (qt, r, c)
+    ch.free()
+
+
+# both one-launch Q8_0 kernels around their bound, half tiles, batches
+@pytest.mark.parametrize("rows,cols", [(1, 32), (9, 544), (7, 8192), (33, 9248), (8192, 96), (8193, 96), (8257, 544),
+                                       (8193, 4096), (8200, 4128)])
+def test_q8_edges(ctx, oracle, rows, cols):
+    print(f"[single] q8_0 {rows}x{cols}", flush=True)
+    w = synth.gen_weights(Q8_0, rows, cols, 31 + rows)
+    x = synth.gen_x(cols, 32 + cols)
+    t = ctx.upload(Q8_0, rows, cols, w)
+    try:
+        acc, xs = ctx.partials(t, x)
+        y = ctx.matmul(t, x)
+    finally:
+        t.free()
+    assert xs == oracle.quantize_act(x)[1]
+    assert acc.shape == (rows, (cols + 63) // 64)
+    assert np.array_equal(bits(y), bits(oracle.matmul(Q8_0, w, x, rows, cols)))

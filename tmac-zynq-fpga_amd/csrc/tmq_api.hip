@@ -116,6 +116,10 @@ struct tmq_chain {
     uint64_t* tail_dev = nullptr;  // tail slots of split groups (zero between launches)
     std::vector<Segment> segs;
     uint64_t weight_bytes = 0;
+    // the chain as one launch (tmq_launch_chain_one): its workgroups in
+    // gmap_dev behind the segments', 0 where the segments are the better way
+    int one_off = 0, one_groups = 0;
+    size_t one_lds = 0;
 };
 
 int tmq_rt_set_device(tmq_ctx* ctx) {
@@ -567,6 +571,42 @@ void plan_segments(std::vector<TmqWork>& works, std::vector<TmqGroupRef>& gmap, 
         sg.ngroups += w.ngroups;
     }
     close();
+}
+
+// Whether the chain's runs take one launch, and its group map (appended).
+// Every workgroup of it quantises its activation again, so the line is drawn
+// by their number: up to two a CU for each launch of a format it replaces.
+// us, one launch against the quantisation and the formats' launches: a layer
+// of Q5_0, Q8_0 and Q6_K products (330 workgroups) 10.6 against 25.5, three
+// 20.0 against 29.5, five 27.3 against 32.8; attn_q, gate and up in Q5_0
+// (184) 6.6 against 10.2, three times 11.6 against 11.1; 896 x 4864 Q6_K
+// (56) 9.2 against 11.8, eight 15.3 against 17.3, Q4_K 12.9 against 15.7;
+// 4864 x 896 Q8_0 (76) 6.5 against 10.4, eight 12.3 against 22.5.
+void plan_one(tmq_chain* ch, std::vector<TmqGroupRef>& gmap, int ncu) {
+    int64_t groups = 0;
+    size_t lds = 0;
+    for (const TmqWork& w : ch->works) {
+        if (!tmq_chain_one_rows(w.t)) return;
+        const int64_t n = w.t.rows_pad / tmq_chain_one_rows(w.t);
+        groups += w.t.type == TMQ_TYPE_Q8_0 ? (n + 1) / 2 : n;  // (four resident where the others are two)
+        lds = std::max(lds, tmq_chain_one_lds(w.t));
+        // a result over an activation: all of them are quantised first
+        for (int a = 0; a < ch->jobs.count; a++) {
+            const uintptr_t x0 = (uintptr_t)ch->jobs.j[a].x, x1 = x0 + sizeof(float) * (size_t)ch->jobs.j[a].n;
+            auto over = [&](const void* p, size_t n) { return p && (uintptr_t)p < x1 && x0 < (uintptr_t)p + n; };
+            const size_t per = w.t.type == TMQ_TYPE_Q8_0 ? (w.t.cols + 63) / 64 : 1;
+            if (over(w.y, sizeof(float) * (size_t)w.t.rows) || over(w.acc, sizeof(int64_t) * per * (size_t)w.t.rows)) return;
+        }
+    }
+    if (groups > 2 * (int64_t)ncu * (int64_t)ch->segs.size()) return;
+    ch->one_off = (int)gmap.size();
+    ch->one_lds = lds;
+    for (size_t i = 0; i < ch->works.size(); i++) {
+        const TmqWork& w = ch->works[i];
+        const int n = w.t.rows_pad / tmq_chain_one_rows(w.t);
+        for (int g = 0; g < n; g++) gmap.push_back(TmqGroupRef{(int32_t)i, g, 0, 0, 0, 1});
+    }
+    ch->one_groups = (int)gmap.size() - ch->one_off;
 }
 
 int launch_segments(const std::vector<Segment>& segs, const void* works_dev, const void* gmap_dev,
@@ -1128,12 +1168,14 @@ int tmq_chain_create(tmq_ctx* ctx, const tmq_desc* descs, int n, tmq_chain** out
     for (int i = 0; i < n; i++) {
         const tmq_desc& d = descs[i];
         ch->works.push_back(make_work(d.weight, (const uint8_t*)ch->act_dev + act_off[act_of[i]], d.y_dev, d.acc_dev));
+        ch->works.back().xf = d.x_dev;
         ch->weight_bytes += d.weight->weight_bytes;
     }
     // TMQ_NOSPLIT=1 (testing): no split groups
     const char* nsp = getenv("TMQ_NOSPLIT");
     int nslots = 0;
     plan_segments(ch->works, gmap, ch->segs, nsp && atoi(nsp) != 0 ? 0 : ctx->ncu, nslots);
+    plan_one(ch, gmap, ctx->ncu);
     e = hipMalloc(&ch->works_dev, sizeof(TmqWork) * ch->works.size());
     if (e == hipSuccess) e = hipMalloc(&ch->gmap_dev, sizeof(TmqGroupRef) * gmap.size());
     if (e == hipSuccess && nslots) e = hipMalloc(&ch->tail_dev, sizeof(uint64_t) * TMQ_TAIL_SLOT_WORDS * nslots);
@@ -1162,6 +1204,12 @@ int tmq_chain_launch(tmq_ctx* ctx, tmq_chain* ch) {
 }
 
 int tmq_chain_run(tmq_ctx* ctx, tmq_chain* ch) {
+    if (ctx && ch && ch->one_groups) {
+        LAUNCH_TRY(tmq_launch_chain_one(ch->jobs, (const TmqWork*)ch->works_dev,
+                                        (const TmqGroupRef*)ch->gmap_dev + ch->one_off, ch->one_groups, ch->one_lds,
+                                        ctx->stream));
+        return 0;
+    }
     int rc = tmq_chain_prepare(ctx, ch);
     return rc ? rc : tmq_chain_launch(ctx, ch);
 }

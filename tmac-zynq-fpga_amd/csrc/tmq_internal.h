@@ -285,6 +285,14 @@ struct TmqGroupRef {
 // split: the segment holds split groups (Q8_0 quarters take dynamic LDS)
 int tmq_launch_chain(int fmt, int clamp, int max_cols, const TmqWork* works_dev, const TmqGroupRef* groups_dev,
                      int total_groups, int split, uint64_t* tail, hipStream_t s);
+// A chain in one launch, its activations quantised by every workgroup (and
+// prepared by the jobs' workgroups): works with xf set, of formats that
+// tmq_chain_one_rows gives the rows of a workgroup for; lds: the largest
+// tmq_chain_one_lds of them.  No result may lie over an activation.
+int tmq_chain_one_rows(const TmqTensorDev& t);
+size_t tmq_chain_one_lds(const TmqTensorDev& t);
+int tmq_launch_chain_one(const TmqActJobs& jobs, const TmqWork* works_dev, const TmqGroupRef* groups_dev, int ngroups,
+                         size_t lds, hipStream_t s);
 // widest Q8_0 rows whose chain groups split into quarters (the quarters'
 // 64-column tile sums, 512 B a tile, meet in LDS)
 #define TMQ_Q8_SPLIT_COLS 4096

@@ -1891,6 +1891,132 @@ __global__ __launch_bounds__(64 * gemv_waves(FMT), FMT == kQ5_0M ? 8 : 1) void c
 }
 
 // -------------------------------------------------- single-launch GEMVs
+// The branches that fold 64-column tiles in order (Q8_0, and matmul_fpga_int16
+// on the rounded weights), the activation's quantisation included.  A
+// workgroup owns 8 rows: lane 8 s + i holds row i and one tile, 8 s of them a
+// wave, so that all tiles of a row are in flight at once (8 a wave; wider
+// rows in batches).  Every workgroup quantises x for itself while its weights
+// are on the way, which costs less than a launch in front.  The tiles'
+// values meet in LDS and 8 lanes fold them in tile order, y += (double)P *
+// x_scale * row_scale (:930-931, :1075-1076).
+constexpr int kTileRows = 8;
+constexpr int kTileX = 272;  // bytes of a tile's x in LDS: 64 int16 xh, 64 xl; 16 more keep tiles off each other's banks
+// waves for all tiles of a row at once, and the dynamic LDS of a workgroup of nw waves
+constexpr int tiles_waves(int cols) { return ((cols + 63) / 64 + 7) / 8 < 16 ? ((cols + 63) / 64 + 7) / 8 : 16; }
+constexpr size_t tiles_lds(int cols, int nw) {
+    return (size_t)((cols + 63) / 64 < 8 * nw ? (cols + 63) / 64 : 8 * nw) * (kTileX + 8 * kTileRows);
+}
+template <bool Q8>
+__device__ __forceinline__ void group_tiles(const TmqWork& w, int g) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t mfma_lds[];
+    __shared__ float red[16];
+    const TmqTensorDev& t = w.t;
+    const int tid = threadIdx.x, nthr = blockDim.x, lane = tid & 63, wave = wave_id(), nw = nthr >> 6;
+    const int n = t.cols, nt = (n + 63) / 64, nc = n >> 3, bt = 8 * nw;  // bt: tiles a batch
+    uint8_t* xb = mfma_lds;
+    double* ps = (double*)(mfma_lds + (size_t)min(nt, bt) * kTileX);  // [tile][kTileRows]
+    const size_t R = t.rows_pad;
+    const int row = lane & (kTileRows - 1), r = g * kTileRows + row;
+    // x of this thread, the first kXR elements in registers
+    constexpr int kXR = 8;
+    float xv[kXR];
+#pragma unroll
+    for (int k = 0; k < kXR; k++) xv[k] = w.xf[min(tid + k * nthr, n - 1)];
+    const float rsf = Q8 ? t.row_scale[r] : t.rs16[r], ri = Q8 ? t.row_inv[r] : 0.0f;
+    const double rs = (double)rsf;
+    // the lane's tile of a batch (slots past the last tile, and the second
+    // half of a half tile, re-read what is there)
+    uint4 v[8];
+    Q8Blk q0, q1;
+    auto load = [&](int tt) {
+        tt = min(tt, nt - 1);
+        if constexpr (Q8) {
+            q0 = q8_load(t, 2 * tt, r);
+            q1 = q8_load(t, min(2 * tt + 1, t.nb - 1), r);
+        } else {
+#pragma unroll
+            for (int c = 0; c < 8; c++) v[c] = ld16(t.pw + ((size_t)min(8 * tt + c, nc - 1) * R + r) * 16);
+        }
+    };
+    const int sub = 8 * wave + (lane >> 3);
+    load(sub);
+    float m = 0.0f;
+#pragma unroll
+    for (int k = 0; k < kXR; k++) m = fmaxf(m, fabsf(xv[k]));
+    for (int j = tid + kXR * nthr; j < n; j += nthr) m = fmaxf(m, fabsf(w.xf[j]));
+    m = tmq_wave_max(m);
+    if (lane == 0) red[wave] = m;
+    __syncthreads();
+    float mm = red[0];
+    for (int i = 1; i < nw; i++) mm = fmaxf(mm, red[i]);
+    const float xs = (mm < 1e-10f) ? 1.0f : mm / 32767.0f;
+    if (w.xs_out && g == 0 && tid == 0) *w.xs_out = xs;
+    float y = 0.0f;
+    for (int tb = 0; tb < nt; tb += bt) {
+        const int te = min(tb + bt, nt);  // this batch's tiles
+        auto put = [&](int j, float x) {
+            const int q = (int)(int16_t)roundf(x / xs), e = j - 64 * tb;
+            int16_t* d = (int16_t*)(xb + (e >> 6) * kTileX) + (e & 63);
+            d[0] = (int16_t)(q >> 8);
+            d[64] = (int16_t)(q & 255);
+        };
+        const int j1 = min(n, 64 * te);
+        int j = 64 * tb + tid;
+        if (tb == 0) {
+#pragma unroll
+            for (int k = 0; k < kXR; k++, j += nthr)
+                if (j < j1) put(j, xv[k]);
+        }
+        for (; j < j1; j += nthr) put(j, w.xf[j]);
+        __syncthreads();
+        const int tt = tb + sub;
+        if (tt < te) {
+            const uint4* X = (const uint4*)(xb + (size_t)sub * kTileX);
+            const int have = min(8, nc - 8 * tt);  // 8-column chunks of the tile (4 or 8)
+            int sh = 0, sl = 0;
+            // int16 weights against xh and xl: |sums| < 2^30 over 64 columns
+            if constexpr (Q8) {
+                auto half = [&](const Q8Blk& k, int h) {
+                    ActN<16> A;
+#pragma unroll
+                    for (int c = 0; c < 4; c++) {
+                        const uint4 a = X[4 * h + c], b = X[8 + 4 * h + c];
+#pragma unroll
+                        for (int i = 0; i < 4; i++) {
+                            A.xh[4 * c + i] = dw_of(a, i);
+                            A.xl[4 * c + i] = dw_of(b, i);
+                        }
+                    }
+                    q8_mac(k, A, 0, ri, sh, sl);
+                };
+                half(q0, 0);
+                if (have == 8) half(q1, 1);
+            } else {
+#pragma unroll
+                for (int c = 0; c < 8; c++) {
+                    if (c >= have) break;
+                    const uint4 h = X[c], l = X[8 + c];
+#pragma unroll
+                    for (int k = 0; k < 4; k++) {
+                        sh = dot2(dw_of(v[c], k), dw_of(h, k), sh);
+                        sl = dot2(dw_of(v[c], k), dw_of(l, k), sl);
+                    }
+                }
+            }
+            const int64_t P = (int64_t)sh * 256 + sl;
+            if (w.acc && r < t.rows) w.acc[(size_t)r * nt + tt] = P;
+            ps[sub * kTileRows + row] = ((double)P * (double)xs) * rs;
+        }
+        if (te < nt) load(te + sub);
+        __syncthreads();
+        if (tid < kTileRows) {
+#pragma unroll 8
+            for (int i = 0; i < te - tb; i++) y = (float)((double)y + ps[i * kTileRows + tid]);
+        }
+    }
+    if (w.y && tid < kTileRows && r < t.rows) store_y(w, r, y);
+}
+
 // x_scale and the MFMA operand bytes of x[0, n) (the layout act_prep_kernel
 // writes), made by the workgroup in LDS: bytes xa, sums over 32 (xsl) and 16
 // (xs16l, unless null) elements, nbx blocks of 32 (those past n zero) and
@@ -1967,33 +2093,182 @@ template <int FMT> __host__ __device__ constexpr int one_part_off(int nbx) {
     return one_xs_off<FMT>(nbx) + nbx * 4 + (FMT == kQ6_KM ? nbx * 8 : 0);
 }
 template <int FMT> __host__ __device__ constexpr int one_lds(int nbx) { return one_part_off<FMT>(nbx) + (kOneWaves + 1) * 64 * 8; }
-template <int FMT, int KX>
-__global__ __launch_bounds__(64 * kOneWaves) void one_kernel(TmqWork w) {
+// (RG 64, Q5_0: 64 rows a workgroup, one a lane, in the one-launch chain)
+template <int FMT, int KX, int RG = 16>
+__device__ __forceinline__ void group_one(const TmqWork& w, int g) {
     extern __shared__ __attribute__((aligned(16))) uint8_t mfma_lds[];
-    tmq_warm_kernargs<sizeof(TmqWork)>();
     const TmqTensorDev& t = w.t;
-    const int g = blockIdx.x, lane = threadIdx.x & 63, n = t.cols, nbx = one_nbx(n);
+    static_assert(RG == 16 || FMT == kQ5_0M, "64-row groups: Q5_0");
+    const int lane = threadIdx.x & 63, n = t.cols, nbx = one_nbx(n);
     uint8_t* xa = mfma_lds + one_ring<FMT>();
     int32_t* xsl = (int32_t*)(mfma_lds + one_xs_off<FMT>(nbx));
     int32_t* xs16l = FMT == kQ6_KM ? xsl + nbx : nullptr;
     int64_t* part = (int64_t*)(mfma_lds + one_part_off<FMT>(nbx));
-    const int r = g * 16 + (lane & 15);
+    const int r = g * RG + (lane & (RG - 1));
     const float inv = t.row_inv[r];
     float xsc = 0.0f;
     auto ready = [&](auto&& prime, int) {
-        xsc = quant_lds<kOneWaves, KX, FMT == kQ5_0M ? kMfmaConst : kKqConst>(w.xf, n, nbx, xa, xsl, xs16l, prime);
+        xsc = quant_lds<kOneWaves, KX, FMT == kQ5_0M ? kMfmaConst : kKqConst>(w.xf, n, RG == 16 ? nbx : t.nb, xa, xsl,
+                                                                              xs16l, prime);
     };
     auto xq = [&](int col) { return quant_elem(xa, col); };
     int64_t tot;
     if constexpr (FMT == kQ5_0M)
-        tot = mfma_q5_rows<kOneWaves, true, true>(t, g, 0, 0, xa, xsl, mfma_lds, part, 0, n, ready, xq);
+        tot = mfma_q5_rows<kOneWaves, true, RG == 16>(t, g, 0, t.nb, xa, xsl, mfma_lds, part, 0, n, ready, xq);
     else
         tot = mfma_kq_rows<FMT == kQ4_KM ? kQ4_K : kQ6_K, true, true, kOneWaves>(t, g, 0, t.nb, xa, xsl, xs16l, mfma_lds,
                                                                                  part, 0, n, ready, xq);
-    if (g == 0 && threadIdx.x == 0) *w.xs_out = xsc;
-    if (threadIdx.x < 16 && r < t.rows) {
+    if (w.xs_out && g == 0 && threadIdx.x == 0) *w.xs_out = xsc;
+    if (threadIdx.x < RG && r < t.rows) {
         if (w.acc) w.acc[r] = tot;
         if (w.y) store_y(w, r, (float)(((double)tot * (double)xsc) / (double)inv));
+    }
+}
+template <int FMT, int KX>
+__global__ __launch_bounds__(64 * kOneWaves) void one_kernel(TmqWork w) {
+    tmq_warm_kernargs<sizeof(TmqWork)>();
+    group_one<FMT, KX>(w, blockIdx.x);
+}
+// Q8_0 tensors of many rows: 64 rows a workgroup, one a lane, the 64-column
+// tiles over its four waves (x from LDS, the same address in every lane),
+// the next tile's weights on the way while one is multiplied.  2374
+// rows x 896, a call: 16000 21.5 us (two launches of 256-row workgroups, a
+// wave a lane's whole row) -> 5.8 (group_tiles 8.1), 65536 22.9 -> 12.9.
+constexpr int kQ8WideCols = 4096;  // (48 KiB of LDS)
+__host__ __device__ constexpr int q8_wide_lds(int cols) { return ((cols + 63) / 64) * (256 + 512); }
+template <int NW>
+__device__ __forceinline__ void group_q8_wide(const TmqWork& w, int g) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t mfma_lds[];
+    __shared__ float red[NW];
+    const TmqTensorDev& t = w.t;
+    const int tid = threadIdx.x, lane = tid & 63, wave = wave_id();
+    const int n = t.cols, nt = (n + 63) / 64, r = g * 64 + lane;
+    double* ps = (double*)(mfma_lds + nt * 256);  // [tile][64]
+    constexpr int kXR = 4;
+    float xv[kXR];
+#pragma unroll
+    for (int k = 0; k < kXR; k++) xv[k] = w.xf[min(tid + 64 * NW * k, n - 1)];
+    const float ri = t.row_inv[r];
+    const double rs = (double)t.row_scale[r];
+    struct Tile {
+        Q8Blk q0, q1;
+    } A, B;
+    auto load = [&](Tile& k, int tt) {
+        tt = min(tt, nt - 1);
+        k.q0 = q8_load(t, 2 * tt, r);
+        k.q1 = q8_load(t, min(2 * tt + 1, t.nb - 1), r);
+    };
+    load(A, wave);
+    float m = 0.0f;
+#pragma unroll
+    for (int k = 0; k < kXR; k++) m = fmaxf(m, fabsf(xv[k]));
+    for (int j = tid + 64 * NW * kXR; j < n; j += 256) m = fmaxf(m, fabsf(w.xf[j]));
+    m = tmq_wave_max(m);
+    if (lane == 0) red[wave] = m;
+    __syncthreads();
+    float mm = red[0];
+#pragma unroll
+    for (int i = 1; i < NW; i++) mm = fmaxf(mm, red[i]);
+    const float xs = (mm < 1e-10f) ? 1.0f : mm / 32767.0f;
+    if (w.xs_out && g == 0 && tid == 0) *w.xs_out = xs;
+    auto put = [&](int j, float x) {
+        const int q = (int)(int16_t)roundf(x / xs);
+        int16_t* d = (int16_t*)(mfma_lds + (j >> 6) * 256) + (j & 63);
+        d[0] = (int16_t)(q >> 8);
+        d[64] = (int16_t)(q & 255);
+    };
+    int j = tid;
+#pragma unroll
+    for (int k = 0; k < kXR; k++, j += 64 * NW)
+        if (j < n) put(j, xv[k]);
+    for (; j < n; j += 64 * NW) put(j, w.xf[j]);
+    __syncthreads();
+    auto mac = [&](const Tile& k, int tt) {
+        const uint4* X = (const uint4*)(mfma_lds + tt * 256);
+        int sh = 0, sl = 0;
+        auto half = [&](const Q8Blk& q, int h) {
+            ActN<16> a;
+#pragma unroll
+            for (int c = 0; c < 4; c++) {
+                const uint4 u = X[4 * h + c], v = X[8 + 4 * h + c];
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    a.xh[4 * c + i] = dw_of(u, i);
+                    a.xl[4 * c + i] = dw_of(v, i);
+                }
+            }
+            q8_mac(q, a, 0, ri, sh, sl);
+        };
+        half(k.q0, 0);
+        if (2 * tt + 1 < t.nb) half(k.q1, 1);
+        const int64_t P = (int64_t)sh * 256 + sl;
+        if (w.acc && r < t.rows) w.acc[(size_t)r * nt + tt] = P;
+        ps[tt * 64 + lane] = ((double)P * (double)xs) * rs;
+    };
+    for (int tt = wave; tt < nt; tt += 2 * NW) {
+        load(B, tt + NW);
+        mac(A, tt);
+        if (tt + NW >= nt) break;
+        load(A, tt + 2 * NW);
+        mac(B, tt + NW);
+    }
+    __syncthreads();
+    if (wave != 0) return;
+    float y = 0.0f;
+#pragma unroll 8
+    for (int i = 0; i < nt; i++) y = (float)((double)y + ps[i * 64 + lane]);
+    if (w.y && r < t.rows) store_y(w, r, y);
+}
+__global__ __launch_bounds__(256) void one_q8_wide_kernel(TmqWork w) {
+    tmq_warm_kernargs<sizeof(TmqWork)>();
+    group_q8_wide<4>(w, blockIdx.x);
+}
+// Q8_0: 8 rows a workgroup (group_tiles)
+__global__ __launch_bounds__(1024) void one_q8_kernel(TmqWork w) {
+    tmq_warm_kernargs<sizeof(TmqWork)>();
+    group_tiles<true>(w, blockIdx.x);
+}
+
+// A whole chain of little work in one launch: first the activation jobs
+// (act_prep_kernel's, for the callers that launch the chain again without
+// quantising), then the descriptors' workgroups (one_rows), which quantise
+// for themselves.  Descriptor -> works[], workgroup -> (descriptor, row
+// group) through groups[].  Held to 128 registers: two workgroups a CU.
+__device__ void act_prep(const TmqActJob& J, float* red);
+__host__ __device__ inline int one_rows(const TmqTensorDev& t) {
+    // Q5_0 of many rows: 64 a workgroup, four times fewer quantisations
+    return t.type == kQ8_0 || (t.type == kQ5_0 && t.rows > 2048 && t.cols <= 128 * kOneWaves) ? 64 : 16;
+}
+template <int KX>
+__device__ __forceinline__ void group_one_kq(const TmqWork& w, int g) {
+    if (w.t.type == kQ4_K)
+        group_one<kQ4_KM, KX>(w, g);
+    else
+        group_one<kQ6_KM, KX>(w, g);
+}
+__global__ __launch_bounds__(64 * kOneWaves, 4) void chain_one_kernel(TmqActJobs jobs, const TmqWork* __restrict__ works,
+                                                                      const TmqGroupRef* __restrict__ groups) {
+    __shared__ float red[kOneWaves + 1];
+    const int b = (int)blockIdx.x - jobs.count;
+    if (b < 0) {
+        act_prep(jobs.j[blockIdx.x], red);
+        return;
+    }
+    const TmqGroupRef ref = groups[b];
+    const TmqWork& w = works[ref.work];
+    if (w.t.type == kQ5_0) {
+        if (one_rows(w.t) == 64)
+            group_one<kQ5_0M, 2, 64>(w, ref.group);
+        else if (w.t.cols <= 128 * kOneWaves)
+            group_one<kQ5_0M, 2>(w, ref.group);
+        else
+            group_one<kQ5_0M, 16>(w, ref.group);
+    } else if (w.t.type == kQ8_0) {
+        group_q8_wide<kOneWaves>(w, ref.group);
+    } else if (w.t.cols <= 640 * kOneWaves) {
+        group_one_kq<10>(w, ref.group);
+    } else {
+        group_one_kq<16>(w, ref.group);
     }
 }
 
@@ -2196,107 +2471,13 @@ __device__ __forceinline__ int64_t i16_tile(const TmqTensorDev& t, const AT& A, 
     return (int64_t)sh * 256 + sl;
 }
 
-// matmul_fpga_int16 (sim/tmac_gguf.cpp:887-940), the activation's
-// quantisation (:890-896) included.  A workgroup owns 8 rows: lane 8 s + i
-// holds row i and one 64-column tile, 8 s of them a wave, so that up to 128
-// tiles are in flight at once and 896 rows give 112 workgroups (a lane per
-// row and one wave per 64 rows left 14 waves to walk 76 tiles one after the
-// other, bound by the latency of each).  Every workgroup quantises x for
-// itself while its weights are on the way, which costs less than a launch in
-// front.  The tiles' values meet in LDS and 8 lanes fold them in tile order,
-// y += (double)result * x_scale * row_scale (:930-931).  Wider rows take
-// kI16Tiles tiles at a time.  A call, launches included: 896 x 4864 180 ->
-// 5.7 us (1.5 TB/s of int16 weights), 4864 x 896 32 -> 4.4, 151936 x 896
-// 74 -> 59 (4.6 TB/s).
-constexpr int kI16Rows = 8, kI16Tiles = 128;
-constexpr int kI16TileX = 272;  // bytes of a tile's x in LDS: 8 columns as 8 xh, 8 xl (int16); 16 keep tiles off each other's banks
-static int i16_waves(int cols) { return ((cols + 63) / 64 + 7) / 8 < 16 ? ((cols + 63) / 64 + 7) / 8 : 16; }
-static size_t i16_lds(int cols) {
-    const int nt = (cols + 63) / 64, b = nt < kI16Tiles ? nt : kI16Tiles;
-    return (size_t)b * (kI16TileX + 8 * kI16Rows);
-}
+// matmul_fpga_int16 (sim/tmac_gguf.cpp:887-940): group_tiles on the rounded
+// weights.  One wave walking the tiles of 64 rows behind a quantisation
+// launch left 14 waves for 896 rows.  A call, launches included: 896 x 4864
+// 180 -> 5.7 us (1.5 TB/s of int16 weights), 4864 x 896 32 -> 4.4, 151936 x
+// 896 74 -> 59 (4.6 TB/s).
 __global__ __launch_bounds__(1024) void i16_gemv_kernel(TmqWork w) {
-    extern __shared__ __attribute__((aligned(16))) uint8_t mfma_lds[];
-    __shared__ float red[16];
-    const TmqTensorDev& t = w.t;
-    const int tid = threadIdx.x, nthr = blockDim.x, lane = tid & 63, wave = wave_id(), nw = nthr >> 6;
-    const int n = t.cols, nt = (n + 63) / 64, nc = n >> 3;
-    uint8_t* xb = mfma_lds;
-    double* ps = (double*)(mfma_lds + (size_t)min(nt, kI16Tiles) * kI16TileX);  // [tile][kI16Rows]
-    const size_t R = t.rows_pad;
-    const int row = lane & (kI16Rows - 1), r = blockIdx.x * kI16Rows + row;
-    // x of this thread, the first kXR elements in registers
-    constexpr int kXR = 8;
-    float xv[kXR];
-#pragma unroll
-    for (int k = 0; k < kXR; k++) xv[k] = w.xf[min(tid + k * nthr, n - 1)];
-    const double rs = (double)t.rs16[r];
-    // the lane's tile of a batch (slots past the last tile re-read it)
-    uint4 v[8];
-    auto load = [&](int tt) {
-        const int c0 = 8 * min(tt, nt - 1);
-#pragma unroll
-        for (int c = 0; c < 8; c++) v[c] = ld16(t.pw + ((size_t)min(c0 + c, nc - 1) * R + r) * 16);
-    };
-    const int sub = 8 * wave + (lane >> 3);
-    load(sub);
-    float m = 0.0f;
-#pragma unroll
-    for (int k = 0; k < kXR; k++) m = fmaxf(m, fabsf(xv[k]));
-    for (int j = tid + kXR * nthr; j < n; j += nthr) m = fmaxf(m, fabsf(w.xf[j]));
-    m = tmq_wave_max(m);
-    if (lane == 0) red[wave] = m;
-    __syncthreads();
-    float mm = red[0];
-    for (int i = 1; i < nw; i++) mm = fmaxf(mm, red[i]);
-    const float xs = (mm < 1e-10f) ? 1.0f : mm / 32767.0f;
-    if (blockIdx.x == 0 && tid == 0) *w.xs_out = xs;
-    float y = 0.0f;
-    for (int tb = 0; tb < nt; tb += kI16Tiles) {
-        const int te = min(tb + kI16Tiles, nt);  // this batch's tiles
-        auto put = [&](int j, float x) {
-            const int q = (int)(int16_t)roundf(x / xs), e = j - 64 * tb;
-            int16_t* d = (int16_t*)(xb + (e >> 6) * kI16TileX + ((e >> 3) & 7) * 32) + (e & 7);
-            d[0] = (int16_t)(q >> 8);
-            d[8] = (int16_t)(q & 255);
-        };
-        const int j1 = min(n, 64 * te);
-        int j = 64 * tb + tid;
-        if (tb == 0) {
-#pragma unroll
-            for (int k = 0; k < kXR; k++, j += nthr)
-                if (j < j1) put(j, xv[k]);
-        }
-        for (; j < j1; j += nthr) put(j, w.xf[j]);
-        __syncthreads();
-        const int tt = tb + sub;
-        if (tt < te) {
-            const uint4* X = (const uint4*)(xb + (size_t)sub * kI16TileX);
-            const int have = min(8, nc - 8 * tt);  // 16-byte chunks of the tile
-            int sh = 0, sl = 0;
-            // 8 weights against xh and xl: |sums| < 2^30 over 64 columns
-#pragma unroll
-            for (int c = 0; c < 8; c++) {
-                if (c >= have) break;
-                const uint4 h = X[2 * c], l = X[2 * c + 1];
-#pragma unroll
-                for (int k = 0; k < 4; k++) {
-                    sh = dot2(dw_of(v[c], k), dw_of(h, k), sh);
-                    sl = dot2(dw_of(v[c], k), dw_of(l, k), sl);
-                }
-            }
-            const int64_t P = (int64_t)sh * 256 + sl;
-            if (w.acc && r < t.rows) w.acc[(size_t)r * nt + tt] = P;
-            ps[sub * kI16Rows + row] = ((double)P * (double)xs) * rs;
-        }
-        if (te < nt) load(te + sub);
-        __syncthreads();
-        if (tid < kI16Rows) {
-#pragma unroll 8
-            for (int i = 0; i < te - tb; i++) y = (float)((double)y + ps[i * kI16Rows + tid]);
-        }
-    }
-    if (w.y && tid < kI16Rows && r < t.rows) store_y(w, r, y);
+    group_tiles<false>(w, blockIdx.x);
 }
 
 // The FP32 loop of `matmul` (sim/tmac_gguf.cpp:488-492): y_r = sum over
@@ -3270,11 +3451,9 @@ __global__ __launch_bounds__(256) void zero_acc_kernel(int64_t* p, size_t n) {
 // ------------------------------------------------------ activation prep
 // sim/tmac_gguf.cpp:1225-1231: x_scale = max|x| (sequential fmaxf; the max
 // is order independent), /32767 unless < 1e-10; xq = (int16)roundf(x/x_scale)
-__global__ __launch_bounds__(1024) void act_prep_kernel(TmqActJobs jobs) {
-    tmq_warm_kernargs<sizeof(TmqActJobs)>();
-    const TmqActJob& J = jobs.j[blockIdx.x];
-    __shared__ float red[16];
-    __shared__ float s_scale;
+// (red: a float a wave, and one more)
+__device__ void act_prep(const TmqActJob& J, float* red) {
+    float& s_scale = red[blockDim.x >> 6];
     const int n = J.n;
     float m = 0.0f;
     for (int j = threadIdx.x; j < n; j += blockDim.x) m = fmaxf(m, fabsf(J.x[j]));
@@ -3329,6 +3508,11 @@ __global__ __launch_bounds__(1024) void act_prep_kernel(TmqActJobs jobs) {
         if ((q & 3) == 0) XS[b] = sum;
     }
     if (threadIdx.x < 8) ((uint32_t*)(XA + 64 * nbx))[threadIdx.x] = threadIdx.x < 4 ? 0u : 0x01010101u;
+}
+__global__ __launch_bounds__(1024) void act_prep_kernel(TmqActJobs jobs) {
+    tmq_warm_kernargs<sizeof(TmqActJobs)>();
+    __shared__ float red[17];
+    act_prep(jobs.j[blockIdx.x], red);
 }
 
 // ------------------------------------------------------------- repack
@@ -4121,7 +4305,8 @@ template <int F, bool C> struct ChainK { static auto fn() { return chain_kernel<
 int tmq_gemv_prepare() {
     const void* fns[] = {(const void*)one_kernel<kQ4_KM, 2>,  (const void*)one_kernel<kQ4_KM, 10>,
                          (const void*)one_kernel<kQ4_KM, 16>, (const void*)one_kernel<kQ6_KM, 2>,
-                         (const void*)one_kernel<kQ6_KM, 10>, (const void*)one_kernel<kQ6_KM, 16>};
+                         (const void*)one_kernel<kQ6_KM, 10>, (const void*)one_kernel<kQ6_KM, 16>,
+                         (const void*)chain_one_kernel};
     const int lds = std::max(one_lds<kQ4_KM>(one_nbx(TMQ_MFMA_MAX_COLS)), one_lds<kQ6_KM>(one_nbx(TMQ_MFMA_MAX_COLS)));
     for (const void* f : fns) {
         const hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
@@ -4129,6 +4314,7 @@ int tmq_gemv_prepare() {
     }
     return 0;
 }
+constexpr int kTilesMaxRows = 8192;
 // One launch of 16-row workgroups up to where 64-row groups fill the chip:
 // the time grows with the weights (0.35 ns a row of 896 Q5_0, 0.62 of 1024
 // and 2.5 of 4096 Q6_K columns) where the two launches' is flat (10 us at
@@ -4137,6 +4323,11 @@ int tmq_gemv_prepare() {
 // Q6_K 20000 x 1024 14.7 against 12.1, 5000 x 4096 11.8 against 19.6.
 bool tmq_gemv_takes_x(const TmqTensorDev& t) {
     const int f = tmq_kernel_fmt(t);
+    // Q8_0: one launch up to 128 M weights (151936 x 896 28.4 us on the wide
+    // kernel, 28.0 on two launches; 100000 x 896 18.6 against 24.9), and
+    // where only 8-row workgroups take the width, up to 49152 rows (32000 x
+    // 4096 46 against 79)
+    if (f == kQ8_0) return t.cols <= kQ8WideCols ? (int64_t)t.rows * t.cols <= 1 << 27 : t.rows <= 49152;
     return (f == kQ5_0M || f == kQ4_KM || f == kQ6_KM) && t.rows <= 16384 && (int64_t)t.rows * t.cols <= 1 << 25;
 }
 int tmq_launch_gemv(const TmqWork& w, hipStream_t s) {
@@ -4146,8 +4337,8 @@ int tmq_launch_gemv(const TmqWork& w, hipStream_t s) {
         if (!w.xf) return (int)hipErrorInvalidValue;
         if (w.path == TMQ_WPATH_INT16) {
             if (!w.t.pw || !w.t.rs16 || !w.xs_out) return (int)hipErrorInvalidValue;
-            hipLaunchKernelGGL(i16_gemv_kernel, dim3(w.t.rows_pad / kI16Rows), dim3(64 * i16_waves(w.t.cols)),
-                               i16_lds(w.t.cols), s, w);
+            const int nw = tiles_waves(w.t.cols);
+            hipLaunchKernelGGL(i16_gemv_kernel, dim3(w.t.rows_pad / kTileRows), dim3(64 * nw), tiles_lds(w.t.cols, nw), s, w);
         } else {
             // above this many rows a lane a row fills the chip (65000 x 896
             // 30 us either way; 151936 x 896 35 us, 69 on f32_rows_kernel;
@@ -4171,6 +4362,16 @@ int tmq_launch_gemv(const TmqWork& w, hipStream_t s) {
         return (int)hipGetLastError();
     }
     const int fmt = tmq_kernel_fmt(w.t);
+    // (4864 x 896 5.2 us against 5.6 on the wide kernel, 16000 x 896 8.1 against 5.8)
+    if (w.xf && fmt == kQ8_0 && w.t.rows > kTilesMaxRows && w.t.cols <= kQ8WideCols) {
+        hipLaunchKernelGGL(one_q8_wide_kernel, dim3(w.t.rows_pad / 64), dim3(256), q8_wide_lds(w.t.cols), s, w);
+        return (int)hipGetLastError();
+    }
+    if (w.xf && fmt == kQ8_0) {
+        const int nw = tiles_waves(w.t.cols);
+        hipLaunchKernelGGL(one_q8_kernel, dim3(w.t.rows_pad / kTileRows), dim3(64 * nw), tiles_lds(w.t.cols, nw), s, w);
+        return (int)hipGetLastError();
+    }
     if (w.xf) {
         const int nbx = one_nbx(w.t.cols), kx = (w.t.cols + 64 * kOneWaves - 1) / (64 * kOneWaves);
         const dim3 grid(w.t.rows_pad / 16), blk(64 * kOneWaves);
@@ -4216,6 +4417,28 @@ int tmq_launch_chain(int fmt, int clamp, int max_cols, const TmqWork* works_dev,
     }
     void* args[] = {&works_dev, &groups_dev, &tail};
     return (int)hipLaunchKernel(k, dim3(total_groups), dim3(64 * gemv_waves(fmt)), args, lds, s);
+}
+
+// rows of a workgroup of the one-launch chain, 0: the format is not in it
+int tmq_chain_one_rows(const TmqTensorDev& t) {
+    const int f = tmq_kernel_fmt(t);
+    const bool in = f == kQ5_0M || f == kQ4_KM || f == kQ6_KM || (f == kQ8_0 && t.cols <= kQ8WideCols);
+    return in ? one_rows(t) : 0;
+}
+size_t tmq_chain_one_lds(const TmqTensorDev& t) {
+    const int nbx = one_nbx(t.cols);
+    switch (tmq_kernel_fmt(t)) {
+    case kQ5_0M: return one_lds<kQ5_0M>(nbx);
+    case kQ4_KM: return one_lds<kQ4_KM>(nbx);
+    case kQ6_KM: return one_lds<kQ6_KM>(nbx);
+    default: return q8_wide_lds(t.cols);
+    }
+}
+int tmq_launch_chain_one(const TmqActJobs& jobs, const TmqWork* works_dev, const TmqGroupRef* groups_dev, int ngroups,
+                         size_t lds, hipStream_t s) {
+    hipLaunchKernelGGL(chain_one_kernel, dim3(jobs.count + ngroups), dim3(64 * kOneWaves), lds, s, jobs, works_dev,
+                       groups_dev);
+    return (int)hipGetLastError();
 }
 
 int tmq_launch_resid_view(const float* x, const TmqDeferred& d, int n, float* out, hipStream_t s) {
