@@ -9,7 +9,7 @@
 #define TMQ_HEAD_DIM 64
 #define TMQ_MAX_POS 3072  // scores + weights, 8 B a position, beside the staged V rows in LDS
 // dynamic LDS of the attention: scores, weights and up to vcap staged V rows
-// (256 B each; all of them up to ~500 positions)
+// (256 B each; all of them up to ~500 positions), or a long context's products
 #define TMQ_ATTN_LDS_MAX (152 * 1024)
 
 
@@ -22,6 +22,11 @@ struct TmqAttnArgs {
     float* ctx;              // out [n_heads*64]
     int32_t n_heads, n_kv, max_pos;
     int32_t vcap;            // V rows staged in LDS at a time (set by the launch)
+    // long contexts: the scores of a head by up to n_split workgroups
+    float* sc;               // [n_heads][max_pos]
+    uint32_t* cnt;           // [n_heads], zero between launches
+    int32_t n_split;         // set by the launch
+    int32_t pad_;
 };
 
 int tmq_launch_attn(const TmqAttnArgs& a, hipStream_t s);

@@ -35,6 +35,148 @@ typedef __attribute__((address_space(3))) float lds_f32;
 // that no phase after the scores waits on memory.  The sums are formed in
 // the reference's order: each score over d ascending, the exp sum and each
 // context dimension over positions ascending, one lane per sum.
+//
+// Long contexts (attn_long, from position kAttnLong): one workgroup's path
+// costs 50 cycles a position -- key and value rows through one CU, the exp
+// sum and the context's multiply-adds in one wave.  There, up to 16
+// workgroups a head (blockIdx.y) take a run of positions' scores each; the
+// last to arrive has them all and goes on alone (nobody waits): the exp sum
+// as speculated segments (seq_sum_spec), the products w[p] * v[p][d] by seven
+// waves, and wave 0 only adds them; 14 cycles a position, most of it the
+// value rows' way into that CU (touching them into its XCD's L2 first
+// changed nothing) and the products' through LDS.  ms a token after a prompt
+// of 512: 1.176 -> 1.139, 900: 1.375 -> 1.214, 2000: 1.975 -> 1.392, 3000:
+// 2.529 -> 1.545; at 450 the one workgroup is ahead, 1.108 against 1.132.
+constexpr int kAttnLong = 480;
+constexpr int kAttnPer = 32, kAttnSeg = 7 * kAttnPer;  // positions of a wave and of a segment of the context sum
+constexpr int kAttnLd = kAttnSeg + 4;                 // (4: the 64 dimensions' float4s on different banks)
+__device__ __forceinline__ void attn_long(const TmqAttnArgs& a, float* lds, const float* vbase, const float* vn, float* red,
+                                          float* s_stat, const uint64_t* tab, const double* ltab, int h, int pos, int active) {
+    const int tid = threadIdx.x, lane = tid & 63, KV = a.n_kv * 64;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int mp4 = (a.max_pos + 3) & ~3;
+    float* ex = lds;               // exp terms / weights (2 mp4 floats)
+    float* prod = lds + 2 * mp4;   // products [2][64][kAttnLd]
+    // this workgroup's scores are at the coherence point (agent-scope
+    // stores) before it counts itself in
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    int* s_cnt = (int*)red;
+    if (tid == 0)
+        s_cnt[0] = (int)__hip_atomic_fetch_add(a.cnt + h, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+    if (s_cnt[0] != active - 1) return;
+    if (tid == 0) __hip_atomic_store(a.cnt + h, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    // every score of the head; the first value rows behind them
+    constexpr int NP = TMQ_MAX_POS / 512;
+    float sv[NP];
+#pragma unroll
+    for (int k = 0; k < NP; k++)
+        sv[k] = __hip_atomic_load(a.sc + (size_t)h * a.max_pos + min(tid + 512 * k, pos), __ATOMIC_RELAXED,
+                                  __HIP_MEMORY_SCOPE_AGENT);
+    const int nseg = pos / kAttnSeg + 1, pw = kAttnPer * (wave - 1);
+    typedef float Rows[kAttnPer];
+    Rows A, B;
+    auto load = [&](Rows& v, int seg) {
+#pragma unroll
+        for (int r = 0; r < kAttnPer; r++) v[r] = vbase[(size_t)min(seg * kAttnSeg + pw + r, pos - 1) * KV + lane];
+    };
+    __builtin_amdgcn_sched_barrier(0);
+    if (wave > 0) {
+        load(A, 0);
+        load(B, 1);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    float m = sv[0];
+#pragma unroll
+    for (int k = 1; k < NP; k++) m = fmaxf(m, sv[k]);  // (positions past the last repeat it)
+    m = tmq_wave_max(m);
+    __syncthreads();
+    if (lane == 0) red[wave] = m;
+    __syncthreads();
+    float mx = red[0];
+#pragma unroll
+    for (int w = 1; w < 8; w++) mx = fmaxf(mx, red[w]);
+    const int n4 = (pos + 4) & ~3, npad = nseg * kAttnSeg;
+#pragma unroll
+    for (int k = 0; k < NP; k++) {
+        const int p = tid + 512 * k;
+        if (p < n4) ex[p] = p <= pos ? tmq_math::tmq_expf_tab(sv[k] - mx, Exp2TabLds{tab}) : 0.0f;
+    }
+    __syncthreads();
+    const float es = seq_sum_spec<8>(ex, n4, prod, (int*)(prod + 512), 0);
+    if (tid == 0) s_stat[0] = tmq_math::tmq_logf_tab(es, LogfTabLds{ltab}) + mx;
+    __syncthreads();
+    const float ls = s_stat[0];
+#pragma unroll
+    for (int k = 0; k < NP + 1; k++) {
+        const int p = tid + 512 * k;
+        if (p < npad) ex[p] = k < NP && p <= pos ? tmq_math::tmq_expf_tab(sv[k < NP ? k : 0] - ls, Exp2TabLds{tab}) : 0.0f;
+    }
+    __syncthreads();
+    // segment k's products are made before barrier k and added after it,
+    // while segment k + 1's go to the other buffer
+    auto barrier = [] { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
+    if (wave > 0) {
+        const float vl = vn[lane];
+        auto make = [&](const Rows& v, int seg) {
+            if (seg >= nseg) return;
+            const int b = seg * kAttnSeg + pw;
+            float* d = prod + (size_t)((seg & 1) * 64 + lane) * kAttnLd + pw;
+            float4 w[kAttnPer / 4];
+#pragma unroll
+            for (int j = 0; j < kAttnPer / 4; j++) w[j] = *(const float4*)(ex + b + 4 * j);
+            __builtin_amdgcn_sched_barrier(0);
+            auto put = [&](auto&& x) {
+#pragma unroll
+                for (int j = 0; j < kAttnPer / 4; j++)
+                    *(float4*)(d + 4 * j) = make_float4(w[j].x * x(4 * j), w[j].y * x(4 * j + 1), w[j].z * x(4 * j + 2),
+                                                        w[j].w * x(4 * j + 3));
+            };
+            // the row of position pos is vn; positions past it 0 (their
+            // weights too): +0, which leaves the sum
+            if (b + kAttnPer <= pos)
+                put([&](int i) { return v[i]; });
+            else
+                put([&](int i) { return b + i < pos ? v[i] : b + i == pos ? vl : 0.0f; });
+        };
+        // (whole rounds of the two sets, so that every wait counts a fixed
+        // number of loads; a segment past the last is not added)
+        for (int k = 0; k < nseg; k += 2) {
+            make(A, k);
+            barrier();
+            load(A, k + 2);
+            __builtin_amdgcn_sched_barrier(0);
+            make(B, k + 1);
+            barrier();
+            load(B, k + 3);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        return;
+    }
+    float acc = 0.0f;
+    for (int k = 0; k < (nseg + 1) / 2 * 2; k++) {
+        barrier();
+        if (k >= nseg) continue;
+        const float4* d = (const float4*)(prod + (size_t)((k & 1) * 64 + lane) * kAttnLd);
+        const int nh = k + 1 < nseg || pos - k * kAttnSeg >= kAttnSeg / 2 ? 2 : 1;  // halves that hold a position
+        for (int hf = 0; hf < nh; hf++) {
+            float4 v[kAttnSeg / 8];
+#pragma unroll
+            for (int i = 0; i < kAttnSeg / 8; i++) v[i] = d[hf * (kAttnSeg / 8) + i];
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int i = 0; i < kAttnSeg / 8; i++) {
+                acc += v[i].x;
+                acc += v[i].y;
+                acc += v[i].z;
+                acc += v[i].w;
+            }
+        }
+    }
+    a.ctx[h * 64 + lane] = acc;
+}
+
 template <bool Q8, bool K8, bool V8>
 __global__ __launch_bounds__(512) void attn_kernel(TmqAttnArgs a) {
     tmq_warm_kernargs<sizeof(TmqAttnArgs)>();
@@ -46,6 +188,8 @@ __global__ __launch_bounds__(512) void attn_kernel(TmqAttnArgs a) {
     __shared__ float qr[64], kr[64], vn[64];
     __shared__ float red[8];
     __shared__ float s_stat[1];
+    __shared__ uint64_t tab[32];
+    __shared__ double ltab[32];
     const int h = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int qpk = a.n_heads / a.n_kv;
@@ -65,12 +209,23 @@ __global__ __launch_bounds__(512) void attn_kernel(TmqAttnArgs a) {
         fk1 = fin_load<K8>(a.k, kv * 64 + 2 * j + 1);
     } else if (tid >= 64 && tid < 128) {
         fv = fin_load<V8>(a.v, kv * 64 + jv);
+    } else if (tid >= 128 && tid < 160) {
+        tab[tid - 128] = tmq_math::exp2_tab(tid - 128);
+    } else if (tid >= 192 && tid < 224) {
+        ltab[tid - 192] = tmq_math::logf_tab(tid - 192);
     }
     const float2 cs = a.rope_cur[j];
     const float* kb = a.kc + kv * 64;
     const float* vbase = a.vc + kv * 64;
-    const int pos = a.state->pos;
+    // (in a scalar register: what is formed from it costs no vector instruction)
+    const int pos = __builtin_amdgcn_readfirstlane(a.state->pos);
     if (a.state->err || pos < 0 || pos >= a.max_pos) return;
+    // a long context: this workgroup's run of positions [p0, p0 + run) of
+    // the `active` workgroups that share the head's
+    const bool lng = a.n_split > 1 && pos >= kAttnLong;
+    const int run = lng ? max(64, ((pos + a.n_split) / a.n_split + 63) & ~63) : pos + 1;
+    const int active = pos / run + 1, p0 = (int)blockIdx.y * run;
+    if ((int)blockIdx.y >= active) return;
     const int vcap = a.vcap;
     // (the q/k/v loads went out with the position's: finished first, so that
     // their registers are free before the key row's)
@@ -84,10 +239,10 @@ __global__ __launch_bounds__(512) void attn_kernel(TmqAttnArgs a) {
     } else if (tid >= 64 && tid < 128) {
         vn[tid - 64] = fin_finish<V8>(a.v, fv, vxs);
     }
-    // the cached key row of position tid (< pos; position pos is kr)
+    // the cached key row of position p0 + tid (< pos; position pos is kr)
     float4 kk[16];
     {
-        const float4* kp = (const float4*)(kb + (size_t)min(tid, max(pos - 1, 0)) * KV);
+        const float4* kp = (const float4*)(kb + (size_t)min(p0 + tid, max(pos - 1, 0)) * KV);
 #pragma unroll
         for (int i = 0; i < 16; i++) kk[i] = kp[i];
     }
@@ -101,19 +256,19 @@ __global__ __launch_bounds__(512) void attn_kernel(TmqAttnArgs a) {
                                              (lds_f32*)(vb + r0 * 64), 16, 0, 0);
         }
     };
-    stage_v(0, min(pos, vcap));
+    if (!lng) stage_v(0, min(pos, vcap));
     __syncthreads();
-    if (tid < 64 && h % qpk == 0) {
+    if (tid < 64 && h % qpk == 0 && blockIdx.y == 0) {
         a.kc[(size_t)pos * KV + kv * 64 + tid] = kr[tid];
         a.vc[(size_t)pos * KV + kv * 64 + tid] = vn[tid];
     }
     // scores[p] = sum_d q[d]*k[p][d] (d ascending), / sqrt(64)
-    for (int p = tid; p <= pos; p += 512) {
+    for (int p = p0 + tid; p <= min(pos, p0 + run - 1); p += 512) {
         float s = 0.0f;
         if (p == pos) {
             for (int d = 0; d < 64; d++) s += qr[d] * kr[d];
         } else {
-            if (p != tid) {
+            if (p != p0 + tid) {
                 const float4* kp = (const float4*)(kb + (size_t)p * KV);
 #pragma unroll
                 for (int i = 0; i < 16; i++) kk[i] = kp[i];
@@ -126,7 +281,14 @@ __global__ __launch_bounds__(512) void attn_kernel(TmqAttnArgs a) {
                 s += qr[4 * i + 3] * kk[i].w;
             }
         }
-        sc[p] = s / 8.0f;
+        if (lng)
+            __hip_atomic_store(a.sc + (size_t)h * a.max_pos + p, s / 8.0f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        else
+            sc[p] = s / 8.0f;
+    }
+    if (lng) {
+        attn_long(a, lds, vbase, vn, red, s_stat, tab, ltab, h, pos, active);
+        return;
     }
     __syncthreads();
     float m = -__builtin_inff();
@@ -137,7 +299,7 @@ __global__ __launch_bounds__(512) void attn_kernel(TmqAttnArgs a) {
     float mx = red[0];
 #pragma unroll
     for (int w = 1; w < 8; w++) mx = fmaxf(mx, red[w]);
-    for (int p = tid; p <= pos; p += 512) ex[p] = tmq_math::tmq_expf(sc[p] - mx);
+    for (int p = tid; p <= pos; p += 512) ex[p] = tmq_math::tmq_expf_tab(sc[p] - mx, Exp2TabLds{tab});
     __syncthreads();
     if (tid == 0) {
         // exp_sum in position order (:1648-1649), 16 terms per batch of LDS reads
@@ -156,11 +318,11 @@ __global__ __launch_bounds__(512) void attn_kernel(TmqAttnArgs a) {
             }
         }
         for (; p <= pos; p++) es += ex[p];
-        s_stat[0] = tmq_math::tmq_logf(es) + mx;
+        s_stat[0] = tmq_math::tmq_logf_tab(es, LogfTabLds{ltab}) + mx;
     }
     __syncthreads();
     const float ls = s_stat[0];
-    for (int p = tid; p <= pos; p += 512) ex[p] = tmq_math::tmq_expf(sc[p] - ls);
+    for (int p = tid; p <= pos; p += 512) ex[p] = tmq_math::tmq_expf_tab(sc[p] - ls, Exp2TabLds{tab});
     // this wave's V copies have landed; the barrier makes every wave's visible
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
@@ -247,7 +409,8 @@ int tmq_attn_vcap(int max_pos) {
     return std::min(all, lim & ~63);
 }
 size_t tmq_attn_lds(int max_pos) {
-    return sizeof(float) * ((size_t)2 * ((max_pos + 3) & ~3) + (size_t)64 * tmq_attn_vcap(max_pos));
+    const size_t one = (size_t)64 * tmq_attn_vcap(max_pos), lng = (size_t)2 * 64 * kAttnLd;
+    return sizeof(float) * ((size_t)2 * ((max_pos + 3) & ~3) + (max_pos > kAttnLong ? std::max(one, lng) : one));
 }
 
 int tmq_attn_prepare() {
@@ -268,12 +431,16 @@ int tmq_launch_attn(const TmqAttnArgs& a0, hipStream_t s) {
         return (int)hipErrorInvalidValue;
     TmqAttnArgs a = a0;
     a.vcap = tmq_attn_vcap(a.max_pos);
+    // (runs of about 192 positions at the end of the cache: workgroups that
+    // a short context leaves idle still cost their dispatch, 0.4 % of a step
+    // at 16 of them a head)
+    a.n_split = a.sc && a.cnt && a.max_pos > kAttnLong ? std::min(16, (a.max_pos + 191) / 192) : 1;
     if (a.vcap < 64) return (int)hipErrorInvalidValue;
     if (!attn_prepared) {
         const int e = tmq_attn_prepare();
         if (e) return e;
     }
-    const dim3 grid(a.n_heads), blk(512);
+    const dim3 grid(a.n_heads, a.n_split), blk(512);
     const size_t lds = tmq_attn_lds(a.max_pos);
     const int code = (a.q.ntiles > 0 ? 4 : 0) | (a.k.ntiles > 0 ? 2 : 0) | (a.v.ntiles > 0 ? 1 : 0);
     switch (code) {

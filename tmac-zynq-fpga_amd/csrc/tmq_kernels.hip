@@ -2686,172 +2686,6 @@ __device__ __forceinline__ EngLds eng_lds(unsigned char* base, int n, int nw, si
     return L;
 }
 
-// sum += the 64 values of a group, in order, in every lane: each lane of a
-// 16-lane row holds four of them (lane i: values 4i .. 4i+3, the same in the
-// four rows), and v_add_f32_dpp row_newbcast:i adds lane i's value of the
-// lane's own row as src0 (src0 + src1 = v + sum, the same rounded value as
-// sum + v).  No LDS traffic inside the chain; a dependent DPP add issues
-// about every 7 cycles.  s_nop 1: the two wait states a DPP read of a VGPR
-// needs after a VALU write of it.
-__device__ __forceinline__ float add64_rowbcast(float4 x, float sum) {
-#define TMQ_RB4(N)                                                                 \
-    "v_add_f32_dpp %0, %1, %0 row_newbcast:" #N " row_mask:0xf bank_mask:0xf\n\t" \
-    "v_add_f32_dpp %0, %2, %0 row_newbcast:" #N " row_mask:0xf bank_mask:0xf\n\t" \
-    "v_add_f32_dpp %0, %3, %0 row_newbcast:" #N " row_mask:0xf bank_mask:0xf\n\t" \
-    "v_add_f32_dpp %0, %4, %0 row_newbcast:" #N " row_mask:0xf bank_mask:0xf\n\t"
-    asm volatile("s_nop 1\n\t" TMQ_RB4(0) TMQ_RB4(1) TMQ_RB4(2) TMQ_RB4(3) TMQ_RB4(4) TMQ_RB4(5) TMQ_RB4(6)
-                     TMQ_RB4(7) TMQ_RB4(8) TMQ_RB4(9) TMQ_RB4(10) TMQ_RB4(11) TMQ_RB4(12) TMQ_RB4(13)
-                         TMQ_RB4(14) TMQ_RB4(15)
-                 : "+v"(sum)
-                 : "v"(x.x), "v"(x.y), "v"(x.z), "v"(x.w));
-#undef TMQ_RB4
-    return sum;
-}
-// Lane i's four values of group g of [i0, i1) (v[i0 + 64g + 4i ..]), +0.0
-// past i1.
-__device__ __forceinline__ float4 seq_group(const float* v, int i0, int i1, int g, int i) {
-    const int b = i0 + 64 * g + 4 * i;
-    if (b + 4 <= i1) return *(const float4*)(v + b);
-    float4 r = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    if (b + 0 < i1) r.x = v[b + 0];
-    if (b + 1 < i1) r.y = v[b + 1];
-    if (b + 2 < i1) r.z = v[b + 2];
-    return r;
-}
-// Sequential fp32 sum of v[i0..i1) in index order from each lane's `sum`
-// (the reference's loops), by a whole wave (the same i0, i1 in every lane;
-// i0 a multiple of 4), from LDS, in groups of 64 (add64_rowbcast), the next
-// group's values read during the current one's adds.  The values past i1 in
-// the last group are +0.0: adding +0.0 leaves any sum whose sign bit is
-// clear unchanged, which the callers guarantee (v >= 0, starts of
-// non-negative bits).
-__device__ __forceinline__ float seq_chain_lds(const float* v, int i0, int i1, float sum) {
-    const int i = threadIdx.x & 15, ng = (i1 - i0 + 63) >> 6;
-    float4 x = ng > 0 ? seq_group(v, i0, i1, 0, i) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    for (int g = 0; g < ng; g++) {
-        const float4 cur = x;
-        if (g + 1 < ng) x = seq_group(v, i0, i1, g + 1, i);
-        sum = add64_rowbcast(cur, sum);
-    }
-    return sum;
-}
-
-// One DPP move of a double across lanes (lanes the control leaves without a
-// source, or outside ROW_MASK, read 0.0).
-template <int CTRL, int ROW_MASK = 0xf>
-__device__ __forceinline__ double dpp_f64(double v) {
-    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, ROW_MASK, 0xf, false);
-    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, ROW_MASK, 0xf, false);
-    return __hiloint2double(hi, lo);
-}
-// Sum of x over the wave's 64 lanes, complete in lane 63: pairs and quads
-// (quad permutations), rows of 8 and 16 (half-row and row mirrors), then
-// row 0 into row 1 and row 2 into row 3 (row_bcast15), rows 0-1 into row 3
-// (row_bcast31).  VALU lane moves only, no LDS round trips.
-__device__ __forceinline__ double wave_sum_f64(double x) {
-    x += dpp_f64<0xb1>(x);       // quad_perm [1,0,3,2]
-    x += dpp_f64<0x4e>(x);       // quad_perm [2,3,0,1]
-    x += dpp_f64<0x141>(x);      // row_half_mirror
-    x += dpp_f64<0x140>(x);      // row_mirror
-    x += dpp_f64<0x142, 0xa>(x);  // row_bcast15
-    x += dpp_f64<0x143, 0xc>(x);  // row_bcast31
-    return x;
-}
-
-// The same sequential sum of v[0..n) (0 + v[0] + v[1] + ..., each add
-// rounded; n a multiple of 4), by S waves of the workgroup at once (S at
-// most the workgroup's waves); every thread calls it, and the result is
-// returned to the lanes of wave 0.  The range is cut into S segments of L
-// values (whole batches of 64); wave j runs segment j from 64 starting
-// values, lane l from the float whose bits are those of c_j plus l - 32, c_j
-// being the fp64 sum of v[0 .. jL) rounded to float (wave 0 from the exact
-// start, 0).  Wave 0 then walks the segments in order: the exact start of
-// segment j is the result of segment j-1, and the lane that started from
-// those very bits performed exactly the sequential adds of that segment, so
-// its result is taken.  When no lane did (the fp32 chain drifted more than
-// 32 ulps from the fp64 sum, as over long runs of equal values), wave 0 runs
-// the segment again from the exact start.  For v >= 0 the float bits order
-// the values, so the 64 starts are 64 consecutive floats; lane l started
-// from max(0, c_j + l - 32), which for the index l = b - c_j + 32 in
-// [0, 64) of an exact start with bits b is b itself whenever b >= 0 as an
-// integer (a float without its sign bit).  miss != 0 moves every window
-// away (each segment then runs again: a test of that path).  scr: S*64
-// words of LDS, scr_c: S words.
-template <int S>
-__device__ __forceinline__ float seq_sum_spec(const float* v, int n, float* scr, int* scr_c, int miss) {
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int L = ((n + S - 1) / S + 63) & ~63;
-    if (wave < S) {
-        const int j0 = min(n, wave * L), j1 = min(n, j0 + L);
-        // centre: lane l adds the runs of 16 values at 16 l + 1024 i
-        double p = 0.0;
-        for (int base = 16 * lane; base < j0; base += 1024) {
-            float4 q4[4];
-#pragma unroll
-            for (int e = 0; e < 4; e++) q4[e] = *(const float4*)(v + min(base + 4 * e, n - 4));
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-                const float x[4] = {q4[e].x, q4[e].y, q4[e].z, q4[e].w};
-#pragma unroll
-                for (int u = 0; u < 4; u++)
-                    if (base + 4 * e + u < j0) p += (double)x[u];
-            }
-        }
-        const int cb = min(__builtin_amdgcn_readlane((int)__float_as_uint((float)wave_sum_f64(p)), 63), 0x7f800000) +
-                       (miss ? (1 << 20) : 0);
-        const float s0 = __uint_as_float((uint32_t)(wave == 0 ? 0 : max(0, cb + lane - 32)));
-        scr[wave * 64 + lane] = seq_chain_lds(v, j0, j1, s0);
-        if (lane == 0) scr_c[wave] = cb;
-    }
-    __syncthreads();
-    float sum = 0.0f;
-    if (wave == 0) {
-        // the segments' results (lane l holds lane l's) and centres into
-        // registers, all read at once (the empty asm keeps the compiler from
-        // moving each read down to its step), then the walk reads them across
-        // lanes with uniform indices
-        float o[S];
-        int c[S];
-#pragma unroll
-        for (int j = 0; j < S; j++) {
-            o[j] = scr[j * 64 + lane];
-            c[j] = scr_c[j];
-        }
-#pragma unroll
-        for (int j = 0; j < S; j++) {
-            c[j] = __builtin_amdgcn_readfirstlane(c[j]);
-            asm volatile("" : "+v"(o[j]), "+s"(c[j]));
-        }
-        // the exact running sum as bits in a scalar register: a step is a
-        // few scalar instructions and one lane read
-        int sb = __builtin_amdgcn_readfirstlane(__float_as_int(o[0]));  // segment 0: exact in every lane
-#pragma unroll
-        for (int j = 1; j < S; j++) {
-            const int j0 = min(n, j * L), j1 = min(n, j0 + L);
-            if (j0 >= j1) break;
-            // idx = sb - c_j + 32; a hit when idx is in [0, 64) and sb >= 0
-            int nsb, miss, idx;
-            asm volatile(
-                "s_sub_i32 %[i], %[sb], %[c]\n\t"
-                "s_add_i32 %[i], %[i], 32\n\t"
-                "s_cmp_lt_u32 %[i], 64\n\t"
-                "s_cselect_b32 %[m], 0, 1\n\t"
-                "s_cmp_lt_i32 %[sb], 0\n\t"
-                "s_cselect_b32 %[m], 1, %[m]\n\t"
-                "s_and_b32 %[i], %[i], 63\n\t"
-                "v_readlane_b32 %[r], %[o], %[i]"
-                : [r] "=s"(nsb), [m] "=&s"(miss), [i] "=&s"(idx)
-                : [sb] "s"(sb), [c] "s"(c[j]), [o] "v"(o[j])
-                : "scc");
-            sb = __builtin_expect(miss, 0)
-                     ? __builtin_amdgcn_readfirstlane(__float_as_int(seq_chain_lds(v, j0, j1, __int_as_float(sb))))
-                     : nsb;
-        }
-        sum = __int_as_float(sb);
-    }
-    return sum;
-}
-
 // The activation of the launch (TmqEngAct), quantised into L.xh / L.xl over
 // the columns [c0, c1) the workgroup reads (all of them for the modes that
 // need the whole vector); returns x_scale.

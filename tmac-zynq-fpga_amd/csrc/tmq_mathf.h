@@ -130,7 +130,12 @@ TMQ_HD inline double logf_tab(int j) {
 #endif
 }
 
-TMQ_HD inline float tmq_logf(float x) {
+struct LogfTabConst {
+    TMQ_HD double operator()(int j) const { return logf_tab(j); }
+};
+
+template <class Tab>
+TMQ_HD inline float tmq_logf_tab(float x, const Tab& tab) {
     const double Ln2 = 0x1.62e42fefa39efp-1;
     const double A0 = -0x1.00ea348b88334p-2, A1 = 0x1.5575b0be00b6ap-2, A2 = -0x1.ffffef20a4123p-2;
     uint32_t ix = as_u32(x);
@@ -147,7 +152,7 @@ TMQ_HD inline float tmq_logf(float x) {
     const uint32_t iz = ix - (tmp & 0xff800000u);
     float zf;
     memcpy(&zf, &iz, 4);
-    const double invc = logf_tab(2 * i), logc = logf_tab(2 * i + 1);
+    const double invc = tab(2 * i), logc = tab(2 * i + 1);
     const double r = __builtin_fma((double)zf, invc, -1.0);
     const double y0 = __builtin_fma((double)k, Ln2, logc);
     const double r2 = r * r;
@@ -156,6 +161,8 @@ TMQ_HD inline float tmq_logf(float x) {
     y = __builtin_fma(y, r2, y0 + r);
     return (float)y;
 }
+
+TMQ_HD inline float tmq_logf(float x) { return tmq_logf_tab(x, LogfTabConst{}); }
 
 // RoPE factors for positions [0, max_pos), as apply_rope forms them on the
 // host (sim/tmac_gguf.cpp:1531-1535): theta = 1/powf(base, (float)d/head_dim),

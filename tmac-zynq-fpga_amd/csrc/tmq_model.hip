@@ -168,6 +168,8 @@ struct tmq_model {
     int n_cand = 0;
     float *kc = nullptr, *vc = nullptr;
     float2* rope = nullptr;
+    float* attn_sc = nullptr;      // scores of a long context's attention (TmqAttnArgs)
+    uint32_t* attn_cnt = nullptr;  // its arrival counts
     float2* rope_cur = nullptr;  // the current position's RoPE row (written by every qkv launch)
     TmqEngState* state = nullptr;
     int32_t* tokens = nullptr;
@@ -267,6 +269,8 @@ int launch_layers(tmq_model* m, bool dump, float* cap = nullptr) {
         aa.n_heads = c.n_heads;
         aa.n_kv = c.n_kv_heads;
         aa.max_pos = c.max_seq;
+        aa.sc = m->attn_sc;
+        aa.cnt = m->attn_cnt;
         PROF("rope+attention", LAUNCH_TRY(tmq_launch_attn(aa, s)));
         if (cap) HIP_TRY(hipMemcpyAsync(cap + l * per + H, m->ctxv, sizeof(float) * H, hipMemcpyDeviceToDevice, s));
         PROF("attn_output", rc = launch_gemv(m, L.o_l));
@@ -1149,6 +1153,8 @@ int build_model(tmq_model* m, const std::vector<Entry>& ents, int max_seq) {
     place("fvec", 4 * fv.size() + 4);
     place("rope", sizeof(float2) * 32 * (size_t)max_seq);
     place("rope_cur", sizeof(float2) * 32);
+    place("attn_sc", 4 * (size_t)c.n_heads * max_seq);
+    place("attn_cnt", 4 * (size_t)c.n_heads);
     place("kc", 4 * (size_t)L * max_seq * KV);
     place("vc", 4 * (size_t)L * max_seq * KV);
     hipError_t e = hipMalloc(&m->dmem, off);
@@ -1171,12 +1177,15 @@ int build_model(tmq_model* m, const std::vector<Entry>& ents, int max_seq) {
     m->fvec = (float*)(B + lay["fvec"]);
     m->rope = (float2*)(B + lay["rope"]);
     m->rope_cur = (float2*)(B + lay["rope_cur"]);
+    m->attn_sc = (float*)(B + lay["attn_sc"]);
+    m->attn_cnt = (uint32_t*)(B + lay["attn_cnt"]);
     m->kc = (float*)(B + lay["kc"]);
     m->vc = (float*)(B + lay["vc"]);
 
     hipStream_t s = ctx->stream;
     HIP_TRY(hipMemcpyAsync(m->fvec, fv.data(), 4 * fv.size(), hipMemcpyHostToDevice, s));
     HIP_TRY(hipMemsetAsync(m->xs, 0, 4 * 4 * (size_t)L, s));
+    HIP_TRY(hipMemsetAsync(m->attn_cnt, 0, 4 * (size_t)c.n_heads, s));
     HIP_TRY(hipMemsetAsync(m->hid[0], 0, 4 * (size_t)H, s));
     HIP_TRY(hipMemsetAsync(m->hid[1], 0, 4 * (size_t)H, s));
     LAUNCH_TRY(tmq_launch_zero_acc(m->kacc, m->kacc_cap, s));

@@ -24,12 +24,6 @@ typedef int tmq_v4i __attribute__((ext_vector_type(4)));
 typedef int tmq_v16i __attribute__((ext_vector_type(16)));
 typedef __attribute__((address_space(3))) int8_t lds_i8;
 
-// tmq_expf with its 2^(i/32) table in LDS
-struct Exp2TabLds {
-    const uint64_t* p;
-    __device__ uint64_t operator()(int i) const { return p[i]; }
-};
-
 __device__ __forceinline__ tmq_v16i mfma(tmq_v4i a, tmq_v4i b, tmq_v16i c) {
     return __builtin_amdgcn_mfma_i32_32x32x32_i8(a, b, c, 0, 0, 0);
 }
