@@ -134,6 +134,7 @@ struct Prefill {
     int dn_split = 4;
     int o_split = 2;   // attn_output GEMM split over K (finalised by the ffn_norm input)
     int qkv_split = 1; // q/k/v GEMM split over K (finished by pf_qkv_fin)
+    bool tuned = false;  // tiles or splits set in the environment: no few-token kernels
     int tile[4] = {4, 4, 3, 1};  // GEMM workgroup tiles: qkv, o, gate/up, down (tmq_launch_pf_gemm)
     // captured prefills, by prompt length, chunk and the settings the
     // launches read (a capture holds the chunk buffers' addresses: dropped
@@ -367,6 +368,7 @@ int check_state(tmq_model* m) {
 // plane set (rows q | k | v), gate and up another (rows gate | up).
 int pf_build_weights(tmq_model* m) {
     Prefill& P = m->pf;
+    for (const char* n : {"TMQ_PF_TILES", "TMQ_PF_SPLIT_DN", "TMQ_PF_SPLIT_O", "TMQ_PF_SPLIT_QKV"}) P.tuned |= getenv(n) != nullptr;
     P.dn_split = std::max(1, env_int("TMQ_PF_SPLIT_DN", P.dn_split));
     P.o_split = std::max(1, env_int("TMQ_PF_SPLIT_O", P.o_split));
     P.qkv_split = std::max(1, env_int("TMQ_PF_SPLIT_QKV", P.qkv_split));
@@ -445,7 +447,7 @@ int pf_build_buffers(tmq_model* m, int chunk) {
     // split-K sums of the down projection and attn_output, or those of q/k/v
     // followed by the Q8_0 V tiles
     const int KV = c.n_kv_heads * TMQ_HEAD_DIM;
-    const size_t part_n = std::max((size_t)std::max(P.dn_split, P.o_split) * T * H,
+    const size_t part_n = std::max((size_t)std::max(TMQ_PF_FEW_SPLIT, std::max(P.dn_split, P.o_split)) * T * H,
                                    (size_t)P.qkv_split * T * (H + 2 * KV) + (size_t)T * KV * (H / TMQ_PF_CHUNK));
     parts.push_back({(void**)&P.part, 8 * part_n});
     parts.push_back({(void**)&P.max_bits, 4 * (size_t)T});
@@ -531,7 +533,8 @@ int pf_run_chunk(tmq_model* m, int p0, int T, bool last) {
     // resident at once (TMQ_PF_GUQ=0: the separate act kernel); its wait
     // gives up after TMQ_PF_GUQ_SPIN polls
     int gq_tiles = 0;
-    const bool gq = env_int("TMQ_PF_GUQ", 1) != 0 &&
+    const bool few = T <= TMQ_PF_FEW_TOKENS && !P.tuned && env_int("TMQ_PF_GUQ", -1) <= 0;
+    const bool gq = !few && env_int("TMQ_PF_GUQ", 1) != 0 &&
                     tmq_pf_gu_quant_fits(tile_gu, T_pad, I, m->ctx->ncu, &gq_tiles) && gq_tiles <= P.chunk / 32;
     const int gq_words = gq_tiles * (I / 32 + 1);  // (row tiles of any GU tile: at most I / 32)
     const int gq_spin = std::max(0, env_int("TMQ_PF_GUQ_SPIN", 1 << 20));
@@ -571,6 +574,9 @@ int pf_run_chunk(tmq_model* m, int p0, int T, bool last) {
         g.KV = KV;
         return g;
     };
+    auto launch = [&](const TmqPfGemm& g, int tile) { return few ? tmq_launch_pf_gemm_few(g, s) : tmq_launch_pf_gemm(g, tile, s); };
+    const int dn_split = few ? std::min(TMQ_PF_FEW_SPLIT, I / TMQ_PF_CHUNK) : std::min(P.dn_split, I / pf_stage_cols(tile_dn));
+    const int o_split = few ? std::min(TMQ_PF_FEW_SPLIT, H / TMQ_PF_CHUNK) : std::min(P.o_split, H / pf_stage_cols(tile_o));  // at most one split per stage
     auto dn_part = [&](int l) {
         TmqPfPart d{};
         d.part = P.part;
@@ -579,7 +585,7 @@ int pf_run_chunk(tmq_model* m, int p0, int T, bool last) {
         d.xs = P.xs[3];
         d.row_inv = m->layers[l].down->dev.row_inv;
         d.bias = nullptr;
-        d.split = std::min(P.dn_split, I / pf_stage_cols(tile_dn));
+        d.split = dn_split;
         d.ld = H;
         d.K = I;
         d.T_pad = T_pad;
@@ -600,7 +606,7 @@ int pf_run_chunk(tmq_model* m, int p0, int T, bool last) {
         LAUNCH_TRY(tmq_launch_pf_act(a0, s));
         // q, k, v -> RoPE -> q buffer and this layer's caches; split over K,
         // finished by pf_qkv_fin (which also folds Q8_0 V tiles)
-        const int qkv_split = std::min(P.qkv_split, H / pf_stage_cols(tile_qkv));
+        const int qkv_split = few ? 1 : std::min(P.qkv_split, H / pf_stage_cols(tile_qkv));
         TmqPfGemm g = gemm(qkv_split > 1 ? TMQ_PF_QKVS : TMQ_PF_QKV, W.qkv, 0);
         g.split = qkv_split;
         g.nseg = 3;
@@ -614,7 +620,7 @@ int pf_run_chunk(tmq_model* m, int p0, int T, bool last) {
         // (the down projection's sums were consumed above)
         g.part = P.part;
         g.tpart = P.part + (qkv_split > 1 ? (size_t)qkv_split * T_pad * (H + 2 * KV) : 0);
-        LAUNCH_TRY(tmq_launch_pf_gemm(g, tile_qkv, s));
+        LAUNCH_TRY(launch(g, tile_qkv));
         if (qkv_split > 1 || Y.v->dev.type == TMQ_TYPE_Q8_0) {
             TmqPfQkvFin f{};
             f.part = qkv_split > 1 ? P.part : nullptr;
@@ -653,11 +659,10 @@ int pf_run_chunk(tmq_model* m, int p0, int T, bool last) {
         // attn_output, split over K; the residual and the finalisation go
         // with the ffn_norm input
         LAUNCH_TRY(tmq_launch_pf_act(act(TMQ_PF_PLAIN, 1, P.ctx, nullptr, H), s));
-        const int o_split = std::min(P.o_split, H / pf_stage_cols(tile_o));  // at most one split per stage
         g = gemm(TMQ_PF_PART, W.o, 1);
         g.split = o_split;
         g.part = P.part;
-        LAUNCH_TRY(tmq_launch_pf_gemm(g, tile_o, s));
+        LAUNCH_TRY(launch(g, tile_o));
         // residual + attn_output, ffn_norm, gate/up + SwiGLU
         TmqPfAct a2 = act(TMQ_PF_RESID_NORM, 2, P.x0, m->fvec + Y.ffn_norm, H);
         a2.d1.part = P.part;
@@ -695,7 +700,7 @@ int pf_run_chunk(tmq_model* m, int p0, int T, bool last) {
             g.gq_spin = gq_spin;
             g.gq_ntiles = gq_tiles;
         }
-        LAUNCH_TRY(tmq_launch_pf_gemm(g, tile_gu, s));
+        LAUNCH_TRY(launch(g, tile_gu));
         if (!gq) {
             TmqPfAct a3 = act(TMQ_PF_SILU, 3, P.s, nullptr, I);
             a3.max_bits = P.max_bits;
@@ -703,9 +708,9 @@ int pf_run_chunk(tmq_model* m, int p0, int T, bool last) {
         }
         // down projection, split over K; finalised by the next layer's input
         g = gemm(TMQ_PF_PART, W.dn, 3);
-        g.split = std::min(P.dn_split, I / pf_stage_cols(tile_dn));
+        g.split = dn_split;
         g.part = P.part;
-        LAUNCH_TRY(tmq_launch_pf_gemm(g, tile_dn, s));
+        LAUNCH_TRY(launch(g, tile_dn));
     }
     if (last) {
         const Layer& Z = m->layers[L - 1];
@@ -751,7 +756,7 @@ int pf_prompt(tmq_model* m, int n, int* done) {
         *done = lim;
         return 0;
     }
-    const int guq = env_int("TMQ_PF_GUQ", 1), spin = env_int("TMQ_PF_GUQ_SPIN", 1 << 20);
+    const int guq = env_int("TMQ_PF_GUQ", -1), spin = env_int("TMQ_PF_GUQ_SPIN", 1 << 20);
     hipGraphExec_t ge = nullptr;
     for (const auto& g : P.graphs)
         if (g.lim == lim && g.chunk == chunk && g.guq == guq && g.spin == spin) ge = g.g;

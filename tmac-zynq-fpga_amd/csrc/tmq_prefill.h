@@ -217,6 +217,15 @@ int tmq_launch_pf_act(const TmqPfAct& a, hipStream_t s);
 // 3 = 64 x 128 with two stage buffers (three workgroups per CU), 4 = 64 x 64
 // with K split in halves between the workgroup's waves (K a multiple of 128)
 int tmq_launch_pf_gemm(const TmqPfGemm& g, int tile, hipStream_t s);
+// the same for few tokens (QKV, GU without the quantising epilogue, PART).
+// Chunks of up to TMQ_PF_FEW_TOKENS take it for all four GEMMs (a prompt of
+// 24 layers, ms: 37 tokens 2.33 -> 1.83, 96 2.37 -> 1.91, 128 2.39 -> 2.11,
+// 160 2.45 -> 2.29, 200 2.52 -> 2.48, 256 2.53 -> 2.56), attn_output and down
+// split over K in TMQ_PF_FEW_SPLIT (down in 3: +0.03 ms, in 2: +0.08; more
+// parts than 4 leave pf_act_kernel's batched path).
+#define TMQ_PF_FEW_TOKENS 192
+#define TMQ_PF_FEW_SPLIT 4
+int tmq_launch_pf_gemm_few(const TmqPfGemm& g, hipStream_t s);
 // Whether every workgroup of a GU launch over T_pad tokens (tile, gu_rows)
 // is resident at once on ncu CUs (the quantising epilogue's wait needs it);
 // the token tiles of the launch in *ntiles.

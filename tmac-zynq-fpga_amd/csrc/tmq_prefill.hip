@@ -619,6 +619,231 @@ __global__ __launch_bounds__(256, TILE == 1 ? 2 : TILE == 3 ? 3 : 1) void pf_gem
     }
 }
 
+// The GEMM of a prompt of few tokens.  With one or two token blocks a launch
+// of pf_gemm_kernel is a few dozen workgroups whose waves mostly hold padding
+// and walk K a stage at a time, each stage a barrier and a memory round trip
+// (gate/up of 37 tokens 28 us, of 512 35 us).  Here a workgroup takes two row
+// blocks by one token block and its four waves a quarter of K each: every
+// wave loads its own fragments into registers, R column steps ahead, and
+// meets the others only after its K range, in LDS: wave q then finishes
+// elements 4q .. 4q+3 of every accumulator, four consecutive rows a lane.
+// Bound by the weight planes' way into the CUs: gate/up of 37 tokens 10.9 us
+// (8.7 MB of planes, 0.8 TB/s) and 6.1 for the quantisation it leaves to
+// pf_act_kernel.  (Two token blocks a workgroup: 256 registers were not
+// enough, 2.14 ms against 1.83 for the 37 tokens.)
+template <int MODE>
+__global__ __launch_bounds__(256, MODE == TMQ_PF_QKV ? 1 : 2) void pf_gemm_few_kernel(TmqPfGemm g) {
+    tmq_warm_kernargs<sizeof(TmqPfGemm)>();
+    constexpr int R = 4, NTB = 1;
+    __shared__ int red[4][3 * 16][64];  // (a row block at a time: two workgroups a CU)
+    __shared__ uint64_t c_tab[32];
+    __shared__ float smax[4][32];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int bx = blockIdx.x, bz = blockIdx.z, tb0 = blockIdx.y * NTB;
+    auto rblk = [&](int i) -> int { return MODE == TMQ_PF_GU ? i * (g.gu_rows >> 5) + bx : 2 * bx + i; };
+    // whole 64-column tiles a wave (the Q8_0 sums are per tile)
+    const int nks = g.K >> 5, nt = g.K >> 6;
+    const int a0 = bz * nt / g.split, an = (bz + 1) * nt / g.split - a0;
+    const int s0 = 2 * (a0 + wave * an / 4), s1 = 2 * (a0 + (wave + 1) * an / 4);
+    int si = 0;
+    if (MODE == TMQ_PF_QKV) {
+        const int r0 = rblk(0) * 32;
+        if (g.nseg > 1 && r0 >= g.seg[1].row0) si = 1;
+        if (g.nseg > 2 && r0 >= g.seg[2].row0) si = 2;
+    }
+    const TmqPfSeg S = si == 0 ? g.seg[0] : si == 1 ? g.seg[1] : g.seg[2];
+    const bool q8 = MODE == TMQ_PF_QKV && S.q8;
+    // the epilogue's row and token terms (they arrive during the K loop):
+    // rows 8 wave + 4 (lane / 32) .. + 3 of each row block
+    const int r4 = 8 * wave + 4 * (lane >> 5);
+    float4 inv4[2], bias4[2];
+    int4 rw4[2];
+    float4 cs4[NTB][2];
+    float xs_raw[NTB];
+    int32_t tx_raw[NTB];
+    const bool hasb = MODE == TMQ_PF_QKV && S.bias != nullptr;
+    if (MODE != TMQ_PF_PART && !q8) {
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            const TmqPfSeg Sg = MODE == TMQ_PF_GU ? g.seg[i] : S;
+            const int row = rblk(i) * 32 + r4, rr = row - Sg.row0;
+            inv4[i] = *(const float4*)(Sg.row_inv + rr);
+            rw4[i] = *(const int4*)(g.rw_t + row);
+            if (hasb) bias4[i] = *(const float4*)(Sg.bias + rr);
+#pragma unroll
+            for (int j = 0; j < NTB; j++)
+                if (MODE == TMQ_PF_QKV && si != 2)
+                    cs4[j][i] = *(const float4*)(g.rope + (size_t)(g.p0 + min((tb0 + j) * 32 + (lane & 31), g.T - 1)) * 32 +
+                                                 ((rr & 63) >> 1));
+        }
+#pragma unroll
+        for (int j = 0; j < NTB; j++) {
+            xs_raw[j] = g.xs[(tb0 + j) * 32 + (lane & 31)];
+            tx_raw[j] = g.tx_t[(tb0 + j) * 32 + (lane & 31)];
+        }
+    }
+    if (MODE == TMQ_PF_GU && threadIdx.x < 32) c_tab[threadIdx.x] = tmq_math::exp2_tab(threadIdx.x);
+
+    struct Step {
+        tmq_v4i w[2][2], x[NTB][2];
+    } st[R];
+    // column step s (steps past the wave's last re-read it)
+    auto load = [&](Step& k, int s) {
+        s = min(s, max(s1, 1) - 1);
+#pragma unroll
+        for (int d = 0; d < 2; d++) {
+#pragma unroll
+            for (int i = 0; i < 2; i++)
+                k.w[i][d] = *(const tmq_v4i*)(g.w + (((size_t)rblk(i) * nks + s) * 2 + d) * 1024 + lane * 16);
+#pragma unroll
+            for (int j = 0; j < NTB; j++)
+                k.x[j][d] = *(const tmq_v4i*)(g.x + (((size_t)(tb0 + j) * nks + s) * 2 + d) * 1024 + lane * 16);
+        }
+    };
+    tmq_v16i acc[2][NTB][3];
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int j = 0; j < NTB; j++)
+#pragma unroll
+            for (int d = 0; d < 3; d++) acc[i][j][d] = tmq_v16i{};
+    static_for<R>([&](auto bc) { load(st[decltype(bc)::value], s0 + decltype(bc)::value); });
+    auto kloop = [&](auto q8c) {
+        constexpr bool Q8 = decltype(q8c)::value;
+        for (int sb = s0; sb < s1; sb += R)
+            static_for<R>([&](auto bc) {
+                constexpr int b = decltype(bc)::value;
+                Step& k = st[b];
+                if (sb + b < s1) {
+#pragma unroll
+                    for (int j = 0; j < NTB; j++)
+#pragma unroll
+                        for (int i = 0; i < 2; i++) {
+                            acc[i][j][0] = mfma(k.w[i][0], k.x[j][0], acc[i][j][0]);
+                            acc[i][j][1] = mfma(k.w[i][0], k.x[j][1], acc[i][j][1]);
+                            acc[i][j][2] = mfma(k.w[i][1], k.x[j][1], acc[i][j][2]);
+                            acc[i][j][1] = mfma(k.w[i][1], k.x[j][0], acc[i][j][1]);
+                        }
+                    if (Q8 && (b & 1)) {
+                        // the 64-column tile just completed (R and s0 even)
+                        const int tile = (sb + b) >> 1;
+#pragma unroll
+                        for (int j = 0; j < NTB; j++) {
+                            const int t = (tb0 + j) * 32 + (lane & 31);
+#pragma unroll
+                            for (int i = 0; i < 2; i++) {
+                                int64_t* out = g.tpart + ((size_t)tile * S.rows + rblk(i) * 32 - S.row0) * g.T_pad + t;
+#pragma unroll
+                                for (int v = 0; v < 16; v++)
+                                    out[(size_t)blk_row(v, lane) * g.T_pad] = 65536 * (int64_t)acc[i][j][0][v] +
+                                                                               256 * (int64_t)acc[i][j][1][v] +
+                                                                               (int64_t)acc[i][j][2][v];
+#pragma unroll
+                                for (int d = 0; d < 3; d++) acc[i][j][d] = tmq_v16i{};
+                            }
+                        }
+                    }
+                }
+                load(k, sb + b + R);
+            });
+    };
+    if (q8) {
+        kloop(std::integral_constant<bool, true>{});
+        return;  // pf_qkv_fin_kernel finishes these rows
+    }
+    kloop(std::integral_constant<bool, false>{});
+
+#pragma unroll
+    for (int j = 0; j < NTB; j++) {
+        int sum[2][3][4];
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            if (i) __syncthreads();  // the first block's sums are read
+#pragma unroll
+            for (int d = 0; d < 3; d++)
+#pragma unroll
+                for (int v = 0; v < 16; v++) red[wave][d * 16 + v][lane] = acc[i][j][d][v];
+            __syncthreads();
+#pragma unroll
+            for (int d = 0; d < 3; d++)
+#pragma unroll
+                for (int k = 0; k < 4; k++) {
+                    const int e = d * 16 + 4 * wave + k;
+                    sum[i][d][k] = red[0][e][lane] + red[1][e][lane] + red[2][e][lane] + red[3][e][lane];
+                }
+        }
+        const int t = (tb0 + j) * 32 + (lane & 31);
+        const bool live = t < g.T;
+        if (MODE == TMQ_PF_PART) {
+            if (!live) continue;
+#pragma unroll
+            for (int i = 0; i < 2; i++) {
+                int64_t o[4];
+#pragma unroll
+                for (int k = 0; k < 4; k++)
+                    o[k] = 65536 * (int64_t)sum[i][0][k] + 256 * (int64_t)sum[i][1][k] + (int64_t)sum[i][2][k];
+                int64_t* dst = g.part + ((size_t)bz * g.T_pad + t) * g.rows + rblk(i) * 32 + r4;
+                *(longlong2*)dst = longlong2{o[0], o[1]};
+                *(longlong2*)(dst + 2) = longlong2{o[2], o[3]};
+            }
+            continue;
+        }
+        // finalised as in pf_gemm_kernel (sim/tmac_gguf.cpp:1303-1305)
+        const double xs = (double)xs_raw[j], tc = (double)(128 * (int64_t)tx_raw[j] + 16384 * (int64_t)g.K);
+        float o[2][4];
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            const float iv[4] = {inv4[i].x, inv4[i].y, inv4[i].z, inv4[i].w};
+            const int rw[4] = {rw4[i].x, rw4[i].y, rw4[i].z, rw4[i].w};
+            const float bv[4] = {bias4[i].x, bias4[i].y, bias4[i].z, bias4[i].w};
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                const double a = digits_f64(sum[i][0][k], sum[i][1][k], sum[i][2][k], tc + (double)(128 * rw[k]));
+                o[i][k] = (float)((a * xs) / (double)iv[k]);
+                if (hasb) o[i][k] = o[i][k] + bv[k];
+            }
+        }
+        if (MODE == TMQ_PF_QKV) {
+            if (!live) continue;
+#pragma unroll
+            for (int i = 0; i < 2; i++) {
+                const int rr = rblk(i) * 32 + r4 - S.row0;
+                if (si != 2) {
+                    // apply_rope (sim/tmac_gguf.cpp:1537-1539)
+                    const float4 cs = cs4[j][i];
+                    const float a = o[i][0], b = o[i][1], c = o[i][2], d = o[i][3];
+                    o[i][0] = a * cs.x - b * cs.y;
+                    o[i][1] = a * cs.y + b * cs.x;
+                    o[i][2] = c * cs.z - d * cs.w;
+                    o[i][3] = c * cs.w + d * cs.z;
+                }
+                float* dst = si == 0   ? g.q_out + (size_t)t * g.H + rr
+                             : si == 1 ? g.kc + (size_t)(g.p0 + t) * g.KV + rr
+                                       : g.vc + (size_t)(g.p0 + t) * g.KV + rr;
+                *(float4*)dst = make_float4(o[i][0], o[i][1], o[i][2], o[i][3]);
+            }
+        } else {
+            // SwiGLU (:459-461) and the token's largest |value| in this workgroup
+            float s[4], m = 0.0f;
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                s[k] = (o[0][k] / (1.0f + tmq_math::tmq_expf_tab(-o[0][k], Exp2TabLds{c_tab}))) * o[1][k];
+                m = fmaxf(m, fabsf(s[k]));
+            }
+            if (live) *(float4*)(g.s_out + (size_t)t * g.gu_rows + bx * 32 + r4) = make_float4(s[0], s[1], s[2], s[3]);
+            m = fmaxf(m, __shfl_xor(m, 32));
+            if (lane < 32) smax[wave][lane] = m;
+            __syncthreads();
+            if (wave == 0 && live && lane < 32)
+                __hip_atomic_fetch_max(g.max_bits + t,
+                                       __builtin_bit_cast(uint32_t, fmaxf(fmaxf(smax[0][lane], smax[1][lane]),
+                                                                          fmaxf(smax[2][lane], smax[3][lane]))),
+                                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+    }
+}
+
 // Attention of token t (position P = p0 + t) for the query heads of KV
 // head g: the decode engine's chains (attn_kernel) per query -- scores
 // summed over d in order and /8, max, exp terms summed over positions in
@@ -1018,6 +1243,33 @@ bool tmq_pf_gu_quant_fits(int tile, int T_pad, int gu_rows, int ncu, int* ntiles
     return false;  // (tile 4 takes no GU launch)
 }
 
+template <int MODE>
+static int launch_few(const TmqPfGemm& g, hipStream_t s) {
+    const dim3 grid(g.rows / 64, (g.T + 31) / 32, g.split);
+    hipLaunchKernelGGL((pf_gemm_few_kernel<MODE>), grid, dim3(256), 0, s, g);
+    return (int)hipGetLastError();
+}
+int tmq_launch_pf_gemm_few(const TmqPfGemm& g, hipStream_t s) {
+    // 64-row tiles inside one tensor, whole 64-column tiles, token rows of
+    // the planes to the end of the last token tile
+    if (g.K <= 0 || g.K % 64 || g.rows % 64 || g.T < 1 || (g.T + 31) / 32 * 32 > g.T_pad || g.split < 1 || g.split > g.K / 64 ||
+        g.gq_d)
+        return (int)hipErrorInvalidValue;
+    if (g.mode != TMQ_PF_PART && g.split != 1) return (int)hipErrorInvalidValue;
+    switch (g.mode) {
+    case TMQ_PF_QKV:
+        for (int i = 0; i < g.nseg; i++)
+            if (g.seg[i].row0 % 64 || (g.seg[i].q8 && !g.tpart)) return (int)hipErrorInvalidValue;
+        return launch_few<TMQ_PF_QKV>(g, s);
+    case TMQ_PF_GU:
+        if (g.gu_rows % 32 || g.rows != 2 * g.gu_rows || !g.s_out || !g.max_bits) return (int)hipErrorInvalidValue;
+        return launch_few<TMQ_PF_GU>(g, s);
+    case TMQ_PF_PART:
+        if (!g.part) return (int)hipErrorInvalidValue;
+        return launch_few<TMQ_PF_PART>(g, s);
+    }
+    return (int)hipErrorInvalidValue;
+}
 int tmq_launch_pf_gemm(const TmqPfGemm& g, int tile, hipStream_t s) {
     // shapes the kernel assumes: 64-column chunks, whole token tiles of the
     // operand planes, whole row tiles (GU: gate/up tiles of NRB/2 blocks),
