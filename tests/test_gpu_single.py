@@ -184,3 +184,20 @@ def test_q8_edges(ctx, oracle, rows, cols):
     assert xs == oracle.quantize_act(x)[1]
     assert acc.shape == (rows, (cols + 63) // 64)
     assert np.array_equal(bits(y), bits(oracle.matmul(Q8_0, w, x, rows, cols)))
+
+
+# host vectors: x read over the bus (up to 1024 x 1024) or brought by a
+# launch, y through the pinned buffer or, above its 4 MiB, copied
+@pytest.mark.parametrize("rows,cols", [(1024, 1024), (1025, 1024), (1024, 1056), (1048577, 32)])
+def test_host_vectors(ctx, oracle, rows, cols):
+    import tmq
+    print(f"[single] host {rows}x{cols}", flush=True)
+    w = synth.gen_weights(Q5_0, rows, cols, 21 + cols)
+    t = ctx.upload(Q5_0, rows, cols, w)
+    try:
+        for seed in (1, 2):
+            x = synth.gen_x(cols, seed)
+            assert np.array_equal(bits(ctx.matmul(t, x)), bits(oracle.matmul(Q5_0, w, x, rows, cols)))
+        assert np.array_equal(bits(ctx.matmul_path(t, x, tmq.PATH_FP32)), bits(oracle.matmul_fp32(Q5_0, w, x, rows, cols)))
+    finally:
+        t.free()

@@ -235,6 +235,8 @@ struct TmqActJobs {
 struct ihipStream_t;
 typedef struct ihipStream_t* hipStream_t;
 int tmq_launch_act_prep(const TmqActJobs& jobs, hipStream_t s);
+// n floats (a multiple of 4, 16-byte aligned) from pinned host memory
+int tmq_launch_stage_x(const float* src, float* dst, int n, hipStream_t s);
 int tmq_launch_repack(int type, const uint8_t* src, const TmqTensorDev& t, hipStream_t s);
 // Q6_K: the MFMA decoder's code plane (TmqTensorDev.pq) from the ql / qh planes
 int tmq_launch_q6_pack(const TmqTensorDev& t, hipStream_t s);

@@ -3282,6 +3282,13 @@ __global__ __launch_bounds__(256) void zero_acc_kernel(int64_t* p, size_t n) {
         __hip_atomic_store(p + i, (int64_t)0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// x[0, n) from pinned host memory into device memory (n % 4 == 0, both 16-byte
+// aligned): a launch where a copy command waits for its own engine.
+__global__ __launch_bounds__(256) void stage_x_kernel(const float4* __restrict__ src, float4* __restrict__ dst, int n4) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i < n4) dst[i] = src[i];
+}
+
 // ------------------------------------------------------ activation prep
 // sim/tmac_gguf.cpp:1225-1231: x_scale = max|x| (sequential fmaxf; the max
 // is order independent), /32767 unless < 1e-10; xq = (int16)roundf(x/x_scale)
@@ -4068,6 +4075,13 @@ __global__ __launch_bounds__(256) void q6_pack_kernel(TmqTensorDev t) {
 int tmq_launch_act_prep(const TmqActJobs& jobs, hipStream_t s) {
     if (jobs.count <= 0) return 0;
     hipLaunchKernelGGL(act_prep_kernel, dim3(jobs.count), dim3(1024), 0, s, jobs);
+    return (int)hipGetLastError();
+}
+
+int tmq_launch_stage_x(const float* src, float* dst, int n, hipStream_t s) {
+    if (n <= 0 || n % 4) return (int)hipErrorInvalidValue;
+    hipLaunchKernelGGL(stage_x_kernel, dim3((unsigned)((n / 4 + 255) / 256)), dim3(256), 0, s, (const float4*)src,
+                       (float4*)dst, n / 4);
     return (int)hipGetLastError();
 }
 

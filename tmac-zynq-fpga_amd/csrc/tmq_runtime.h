@@ -46,11 +46,43 @@ struct TmqDevBuf {
     }
 };
 
+// growable pinned host buffer, at most TMQ_HOST_STAGE_MAX bytes
+#define TMQ_HOST_STAGE_MAX ((size_t)4 << 20)
+// activations up to this length, of tensors of up to this many rows, are read
+// from there by the GEMV's workgroups (896 x 896: 19.7 us a call, 21.3 with a
+// launch that brings x to the device first)
+#define TMQ_HOST_X_ROWS 1024
+#define TMQ_HOST_X_COLS 1024
+struct TmqHostBuf {
+    void* p = nullptr;
+    size_t cap = 0;
+    // false: not available (the caller copies to or from pageable memory)
+    bool ensure(size_t n) {
+        if (n <= cap) return true;
+        if (n > TMQ_HOST_STAGE_MAX) return false;
+        release();
+        const size_t want = n < 65536 ? 65536 : n;
+        if (hipHostMalloc(&p, want, hipHostMallocDefault) != hipSuccess) {
+            (void)hipGetLastError();
+            p = nullptr;
+            return false;
+        }
+        cap = want;
+        return true;
+    }
+    void release() {
+        if (p) (void)hipHostFree(p);
+        p = nullptr;
+        cap = 0;
+    }
+};
+
 struct tmq_ctx {
     int device = 0;
     int ncu = 0;  // compute units of the device
     hipStream_t stream = nullptr;
     TmqDevBuf x, y, act, acc, misc, works, gmap;
+    TmqHostBuf hx, hy;  // host vectors of tmq_matmul*
 };
 
 struct tmq_tensor {
