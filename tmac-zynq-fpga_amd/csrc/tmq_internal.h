@@ -265,6 +265,10 @@ int tmq_launch_rowstat(const TmqTensorDev& t, const float* aux_max_abs, float* r
 // says yes to), from the fp32 activation itself; x_scale goes to *w.xs_out
 // (not FP32).  With w.xf no result may lie over the activation.
 int tmq_launch_gemv(const TmqWork& w, hipStream_t s);
+// FP32 works of up to this many rows run 16 rows a workgroup (the engine's
+// too, but for those that leave argmax candidates), others a lane a row
+#define TMQ_F32_ROWS_MAX 65536
+#define TMQ_F32_ROWS 16
 bool tmq_gemv_takes_x(const TmqTensorDev& t);
 // before the first of them on a device (current): their kernels' LDS limits
 int tmq_gemv_prepare();

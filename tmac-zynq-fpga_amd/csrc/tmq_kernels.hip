@@ -2510,15 +2510,20 @@ __global__ __launch_bounds__(64 * TMQ_WAVES) void f32_gemv_kernel(TmqWork w) {
 // reads in front of them, 7.4 cycles a column (reads kept in flight behind
 // the adds, singly or in two sets of eight, were slower: 7.9-11 cycles).
 // A call: 4864 x 896 23.3 -> 6.2 us, 896 x 4864 122 -> 19.
-constexpr int kF32Rows = 16, kF32Prod = 3, kF32Cols = 128 * kF32Prod;
+constexpr int kF32Rows = TMQ_F32_ROWS, kF32Prod = 3, kF32Cols = 128 * kF32Prod;
 constexpr int kF32Ld = kF32Cols + 4;  // (4: the 16 rows' float4 reads on different banks)
-template <int FMT>
-__global__ __launch_bounds__(64 * (1 + kF32Prod)) void f32_rows_kernel(TmqWork w) {
-    __shared__ __attribute__((aligned(16))) float prod[2][kF32Rows][kF32Ld];
-    __shared__ __attribute__((aligned(16))) float xs[kF32Prod][128];
-    const TmqTensorDev& t = w.t;
+struct F32Lds {
+    float prod[2][kF32Rows][kF32Ld];
+    float xs[kF32Prod][128];
+};
+// rows 16 g .. of t; xat(j): element j of the activation; put(r, sum): row
+// r's result, from lanes 0 .. 15 of wave 0
+template <int FMT, class XAt, class Put>
+__device__ __forceinline__ void f32_rows(const TmqTensorDev& t, int g, F32Lds& L, XAt&& xat, Put&& put) {
+    auto& prod = L.prod;
+    auto& xs = L.xs;
     const int lane = threadIdx.x & 63, wave = wave_id();
-    const int row = lane & (kF32Rows - 1), r0 = blockIdx.x * kF32Rows;
+    const int row = lane & (kF32Rows - 1), r0 = g * kF32Rows;
     const int n = t.cols, nbat = (n + kF32Cols - 1) / kF32Cols;
     // batch k is made before barrier k and added after it, while batch k + 1
     // goes to the other buffer (its batch k - 1 was added before barrier k)
@@ -2532,8 +2537,8 @@ __global__ __launch_bounds__(64 * (1 + kF32Prod)) void f32_rows_kernel(TmqWork w
         // (columns past the row's last block re-read it)
         auto load = [&](Set& s, int k) {
             const int j = kF32Cols * k + 128 * p + lane;
-            s.x0 = w.xf[min(j, n - 1)];
-            s.x1 = w.xf[min(j + 64, n - 1)];
+            s.x0 = xat(min(j, n - 1));
+            s.x1 = xat(min(j + 64, n - 1));
             raw32<FMT>(t, r0 + row, min(kF32Cols * k + off, n - 32), s.raw);
         };
         auto make = [&](const Set& s, int k) {
@@ -2584,7 +2589,14 @@ __global__ __launch_bounds__(64 * (1 + kF32Prod)) void f32_rows_kernel(TmqWork w
             }
         }
     }
-    if (w.y && lane < kF32Rows && r0 + row < t.rows) store_y(w, r0 + row, sum);
+    if (lane < kF32Rows && r0 + row < t.rows) put(r0 + row, sum);
+}
+template <int FMT>
+__global__ __launch_bounds__(64 * (1 + kF32Prod)) void f32_rows_kernel(TmqWork w) {
+    __shared__ __attribute__((aligned(16))) F32Lds L;
+    f32_rows<FMT>(w.t, blockIdx.x, L, [&](int j) { return w.xf[j]; }, [&](int r, float v) {
+        if (w.y) store_y(w, r, v);
+    });
 }
 
 // ------------------------------------------------------------ engine GEMV
@@ -3176,6 +3188,25 @@ __device__ __forceinline__ void eng_group_i16(const TmqEngAct& a, const EngLds& 
 // the launch's fp32 activation o = L.x * red[1] (the rms_norm output
 // fl(fl(x*w)*scale), :447-453, or the input itself).  The rows are final
 // values (TmqDeferred.val); the logits also leave argmax candidates.
+// The FP32 loop of a launch's works (no candidates): 16 rows a workgroup
+// (f32_rows), from the activation the prologue left in LDS.
+template <int NW, bool MULTI>
+__device__ __forceinline__ void eng_group_f32_rows(const TmqEngAct& a, const EngLds& L, const TmqWork& w, int g) {
+    static_assert(NW == 1 + kF32Prod, "f32_rows' waves");
+    __shared__ __attribute__((aligned(16))) F32Lds F;
+    const TmqTensorDev& t = w.t;
+    (void)eng_prologue<NW, eng_norm_segs<NW, kQ8_0, MULTI>()>(a, L, 0, t.cols, [] {});
+    const float sc = L.red[1];
+    auto x = [&](int j) { return L.x[j] * sc; };
+    auto put = [&](int r, float v) { __hip_atomic_store(w.y + r, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
+    switch (t.type) {
+    case kQ8_0: f32_rows<kQ8_0>(t, g, F, x, put); break;
+    case kQ5_0: f32_rows<kQ5_0>(t, g, F, x, put); break;
+    case kQ4_K: f32_rows<kQ4_K>(t, g, F, x, put); break;
+    case kQ6_K: f32_rows<kQ6_K>(t, g, F, x, put); break;
+    }
+}
+
 template <int NW, bool MULTI>
 __device__ __forceinline__ void eng_group_f32(const TmqEngAct& a, const EngLds& L, const TmqWork& w, int g) {
     const TmqTensorDev& t = w.t;
@@ -3201,7 +3232,7 @@ __device__ __forceinline__ void eng_group_f32(const TmqEngAct& a, const EngLds& 
 // kQ8_DIRECT for the logits (Q8_0, one wave per 64 rows, direct output).
 constexpr int kQ8_DIRECT = 108;
 // the other branches of matmul: INT16 K-split / direct, FP32
-constexpr int kI16 = 116, kI16_DIRECT = 117, kF32P = 200;
+constexpr int kI16 = 116, kI16_DIRECT = 117, kF32P = 200, kF32R = 201;  // kF32R: 16-row workgroups
 
 template <int NW, int FMT, bool MULTI>
 __device__ __forceinline__ void eng_dispatch(const TmqEngAct& a, const EngLds& L, const TmqWork& w) {
@@ -3211,6 +3242,7 @@ __device__ __forceinline__ void eng_dispatch(const TmqEngAct& a, const EngLds& L
     else if constexpr (FMT == kI16) eng_group_i16_split<NW, MULTI>(a, L, w, g);
     else if constexpr (FMT == kI16_DIRECT) eng_group_i16<NW>(a, L, w, g);
     else if constexpr (FMT == kF32P) eng_group_f32<NW, MULTI>(a, L, w, g);
+    else if constexpr (FMT == kF32R) eng_group_f32_rows<NW, MULTI>(a, L, w, g);
     else if constexpr (FMT == kQ5_0M || FMT == kQ4_KM || FMT == kQ6_KM) eng_group_mfma<FMT, NW, MULTI>(a, L, w, g);
     else eng_group_k<FMT, NW, MULTI>(a, L, w, g);
 }
@@ -3812,7 +3844,7 @@ __global__ __launch_bounds__(64) void pf_wdigits_kernel(TmqTensorDev t, int8_t* 
     const WDigits S{planes, row0 + r, K};
     int sh = 0, sl = 0;
     const float inv = t.row_inv[r];
-    for (int b = 0; b < t.nb; b++) {
+    for (int b = blockIdx.y; b < t.nb; b += gridDim.y) {
         if constexpr (FMT == kQ8_0) q8_mac(q8_load(t, b, r), S, b, inv, sh, sl);
         else blk_mac<FMT, false>(blk_load<FMT>(t, b, r), S, b, inv, sh, sl);
     }
@@ -4191,7 +4223,7 @@ int tmq_launch_gemv(const TmqWork& w, hipStream_t s) {
             // above this many rows a lane a row fills the chip (65000 x 896
             // 30 us either way; 151936 x 896 35 us, 69 on f32_rows_kernel;
             // 32768 x 896 31 against 17)
-            if (w.t.rows > 65536) {
+            if (w.t.rows > TMQ_F32_ROWS_MAX) {
                 const int g = (w.t.rows_pad / 64 + TMQ_WAVES - 1) / TMQ_WAVES;
                 hipLaunchKernelGGL(f32_gemv_kernel, dim3(g), dim3(64 * TMQ_WAVES), 0, s, w);
                 return (int)hipGetLastError();
@@ -4328,6 +4360,7 @@ static void* eng_kernel_for(int fa, int fb) {
         // the INT16 / FP32 branches (4-wave launches only)
         if (fa == kI16 && fb == kI16) return TMQ_ENG_K(kI16, kI16);
         if (fa == kF32P && fb == kF32P) return TMQ_ENG_K(kF32P, kF32P);
+        if (fa == kF32R && fb == kF32R) return TMQ_ENG_K(kF32R, kF32R);
         if constexpr (MULTI) {
             if (fa == kQ5_0 && fb == kI16) return TMQ_ENG_K(kQ5_0, kI16);
             if (fa == kI16 && fb == kQ8_0) return TMQ_ENG_K(kI16, kQ8_0);
@@ -4347,7 +4380,7 @@ static int eng_resolve(const TmqEngLaunch& l, int waves, void** kernel, size_t* 
     // format of the first and the last work (the others must match the first)
     auto code = [](const TmqWork& w) {
         if (w.path == TMQ_WPATH_INT16) return w.kacc ? kI16 : kI16_DIRECT;
-        if (w.path == TMQ_WPATH_FP32) return kF32P;
+        if (w.path == TMQ_WPATH_FP32) return w.cand || w.t.rows > TMQ_F32_ROWS_MAX ? kF32P : kF32R;
         if (w.t.type == kQ8_0) return w.kacc ? kQ8_0 : kQ8_DIRECT;
         // the MFMA decoders where the tensor carries their planes
         return tmq_kernel_fmt(w.t);
@@ -4439,7 +4472,9 @@ int tmq_launch_check_finite(const TmqTensorDev& t, int* bad, hipStream_t s) {
 // ------------------------------------------------------ prefill operands
 int tmq_launch_pf_wdigits(const TmqTensorDev& t, int8_t* planes, int K, int row0, hipStream_t s) {
     if (t.cols != K || K % TMQ_PF_CHUNK || row0 % 32) return (int)hipErrorInvalidValue;
-    const dim3 grid((t.rows + 63) / 64), blk(64);
+    // (a wave walking a row's blocks one after another was latency: a model's
+    // first prompt 10.3 ms)
+    const dim3 grid((t.rows + 63) / 64, std::min(t.nb, 65535)), blk(64);
     switch (t.type) {
     case kQ5_0: hipLaunchKernelGGL(pf_wdigits_kernel<kQ5_0>, grid, blk, 0, s, t, planes, K, row0); break;
     case kQ8_0: hipLaunchKernelGGL(pf_wdigits_kernel<kQ8_0>, grid, blk, 0, s, t, planes, K, row0); break;
