@@ -168,6 +168,23 @@ def test_chain_result_over_activation(ctx, oracle):
     ch.free()
 
 
+def test_chain_shared_result(ctx, oracle):
+    """two descriptors of one result: the later format's launch wins, as ever"""
+    import torch
+    shapes = [(Q6_K, 32, 256, 0), (Q5_0, 32, 96, 1)]
+    ch, xs, xh, ys, ws = chain_of(ctx, torch, shapes)
+    y = ys[0].data_ptr()
+    ch.free()
+    import tmq
+    ts = [ctx.upload(qt, r, c, w) for (qt, r, c, _), w in zip(shapes, ws)]
+    ch = tmq.Chain(ctx, [(ts[0], xs[0].data_ptr(), y, None, 1, 32, 1), (ts[1], xs[1].data_ptr(), y, None, 4, 8, 1)])
+    for _ in range(5):
+        ch.run()
+    ctx.sync()
+    assert np.array_equal(bits(ys[0].cpu().numpy()), bits(oracle.matmul(Q6_K, ws[0], xh[0], 32, 256)))
+    ch.free()
+
+
 # both one-launch Q8_0 kernels around their bound, half tiles, batches
 @pytest.mark.parametrize("rows,cols", [(1, 32), (9, 544), (7, 8192), (33, 9248), (8192, 96), (8193, 96), (8257, 544),
                                        (8193, 4096), (8200, 4128)])

@@ -585,6 +585,16 @@ void plan_segments(std::vector<TmqWork>& works, std::vector<TmqGroupRef>& gmap, 
 void plan_one(tmq_chain* ch, std::vector<TmqGroupRef>& gmap, int ncu) {
     int64_t groups = 0;
     size_t lds = 0;
+    // results that lie over each other: the formats' launches order them
+    std::vector<std::pair<uintptr_t, uintptr_t>> out;
+    for (const TmqWork& w : ch->works) {
+        const size_t per = w.t.type == TMQ_TYPE_Q8_0 ? (w.t.cols + 63) / 64 : 1;
+        if (w.y) out.push_back({(uintptr_t)w.y, (uintptr_t)w.y + sizeof(float) * (size_t)w.t.rows});
+        if (w.acc) out.push_back({(uintptr_t)w.acc, (uintptr_t)w.acc + sizeof(int64_t) * per * (size_t)w.t.rows});
+    }
+    std::sort(out.begin(), out.end());
+    for (size_t i = 1; i < out.size(); i++)
+        if (out[i].first < out[i - 1].second) return;
     for (const TmqWork& w : ch->works) {
         if (!tmq_chain_one_rows(w.t)) return;
         const int64_t n = w.t.rows_pad / tmq_chain_one_rows(w.t);
