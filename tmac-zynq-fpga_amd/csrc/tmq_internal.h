@@ -317,6 +317,8 @@ int tmq_launch_silu(const TmqDeferred& g, const TmqDeferred& u, int n, float* x,
 size_t tmq_eng_lds_bytes(int n, int waves, int fa, int fb);
 // out[i] = x[i] + finalise(d, i), i < n
 int tmq_launch_resid_view(const float* x, const TmqDeferred& d, int n, float* out, hipStream_t s);
+// out[i] = finalise(d, i), i < n, for a tiled product (d.ntiles > 0)
+int tmq_launch_fin_tiles(const TmqDeferred& d, int n, float* out, hipStream_t s);
 // zero n int64 K-split accumulators
 int tmq_launch_zero_acc(int64_t* p, size_t n, hipStream_t s);
 int tmq_launch_tile_q8(const uint8_t* W, const uint16_t* cs, const int16_t* vec, int64_t* out,

@@ -159,6 +159,7 @@ struct tmq_model {
     // residual stream, double buffered: hid[1] = after the attention block's
     // input materialisation (embedding / + down), hid[0] = after + attn_output
     float* hid[2] = {nullptr, nullptr};
+    float* fin[2] = {nullptr, nullptr};  // attn_output / down rows of a tiled product, finalised (tmq_launch_fin_tiles)
     float *ctxv = nullptr, *logits = nullptr, *fvec = nullptr, *dump = nullptr, *view = nullptr;
     int64_t* kacc = nullptr;  // all K-split accumulators of a step
     size_t kacc_n = 0;        // used by the current flags (zeroed per step)
@@ -230,6 +231,23 @@ int launch_gemv(tmq_model* m, const Launch& l) {
     LAUNCH_TRY(tmq_launch_eng_gemv(l.P, l.waves, m->ctx->stream));
     return 0;
 }
+// the same, its H rows finalised into m->fin[k] where they are tile sums
+int launch_gemv_fin(tmq_model* m, const Launch& l, const TmqDeferred& d, int k) {
+    const int rc = launch_gemv(m, l);
+    if (rc || d.ntiles == 0 || d.val) return rc;
+    LAUNCH_TRY(tmq_launch_fin_tiles(d, m->cfg.hidden, m->fin[k], m->ctx->stream));
+    return 0;
+}
+// what the next launch's residual reads of those rows
+TmqDeferred fin_of(const tmq_model* m, const TmqDeferred& d, int k) {
+    if (d.ntiles == 0 || d.val) return d;
+    TmqDeferred f{};
+    f.val = m->fin[k];
+    f.acc = (const int64_t*)f.val;
+    f.row_inv = f.row_scale = f.val;
+    f.xs = d.xs;
+    return f;
+}
 
 // all layers at the current position (forward_all_layers); layer 0's QKV
 // launch also performs process_embedding of tokens[pos].  The step's K-split
@@ -274,7 +292,7 @@ int launch_layers(tmq_model* m, bool dump, float* cap = nullptr) {
         aa.cnt = m->attn_cnt;
         PROF("rope+attention", LAUNCH_TRY(tmq_launch_attn(aa, s)));
         if (cap) HIP_TRY(hipMemcpyAsync(cap + l * per + H, m->ctxv, sizeof(float) * H, hipMemcpyDeviceToDevice, s));
-        PROF("attn_output", rc = launch_gemv(m, L.o_l));
+        PROF("attn_output", rc = launch_gemv_fin(m, L.o_l, L.dout, 0));
         if (rc) return rc;
         PROF(L.fused_gu ? "ffn_norm+gate+up+silu_x_up" : "ffn_norm+gate+up", rc = launch_gemv(m, L.gu));
         if (rc) return rc;
@@ -284,7 +302,7 @@ int launch_layers(tmq_model* m, bool dump, float* cap = nullptr) {
         if (cap)
             HIP_TRY(hipMemcpyAsync(cap + l * per + 3 * (size_t)H, m->silu_x, sizeof(float) * c.inter,
                                    hipMemcpyDeviceToDevice, s));
-        PROF("ffn_down", rc = launch_gemv(m, L.dn));
+        PROF("ffn_down", rc = launch_gemv_fin(m, L.dn, L.dd, 1));
         if (rc) return rc;
         if (dump) LAUNCH_TRY(tmq_launch_resid_view(m->hid[0], L.dd, H, m->dump + (size_t)(l + 1) * H, s));
     }
@@ -920,7 +938,7 @@ int build_launches(tmq_model* m) {
             Y.qkv.P.act.emb = m->emb->dev;
         } else {
             Y.qkv.P.act = recipe(TMQ_ACT_RESID_NORM, m->hid[0], m->fvec + Y.attn_norm, H);
-            Y.qkv.P.act.d1 = m->layers[l - 1].dd;
+            Y.qkv.P.act.d1 = fin_of(m, m->layers[l - 1].dd, 1);
         }
         Y.qkv.P.act.hidden_out = m->hid[1];
         Y.qkv.waves = all_fpga({Y.q, Y.k, Y.v}) ? nw_qkv : 4;
@@ -935,7 +953,7 @@ int build_launches(tmq_model* m) {
         Y.o_l.waves = all_fpga({Y.o}) ? nw_o : 4;
         add_work(Y.o_l, Y.o, ao, xs + 1, kc_o);
         Y.gu.P.act = recipe(TMQ_ACT_RESID_NORM, m->hid[1], m->fvec + Y.ffn_norm, H);
-        Y.gu.P.act.d1 = Y.dout;
+        Y.gu.P.act.d1 = fin_of(m, Y.dout, 0);
         Y.gu.P.act.hidden_out = m->hid[0];
         Y.fused_gu = Y.gu_t && all_fpga({Y.gate, Y.up});
         Y.gu.waves = all_fpga({Y.gate, Y.up}) ? nw_gu : 4;
@@ -962,7 +980,7 @@ int build_launches(tmq_model* m) {
     m->logits_l = Launch{};
     m->logits_l.waves = 4;
     m->logits_l.P.act = recipe(TMQ_ACT_RESID_NORM, m->hid[0], m->out_norm >= 0 ? m->fvec + m->out_norm : nullptr, H);
-    m->logits_l.P.act.d1 = m->layers[L - 1].dd;
+    m->logits_l.P.act.d1 = fin_of(m, m->layers[L - 1].dd, 1);
     {
         TmqWork w = tmq_rt_make_work(m->emb, nullptr, m->logits, nullptr);
         const int g64 = m->emb->dev.rows_pad / 64;
@@ -1148,6 +1166,8 @@ int build_model(tmq_model* m, const std::vector<Entry>& ents, int max_seq) {
     place("hid0", 4 * (size_t)H);
     place("hid1", 4 * (size_t)H);
     place("view", 4 * (size_t)H);
+    place("fin0", 4 * (size_t)H);
+    place("fin1", 4 * (size_t)H);
     place("ctx", 4 * (size_t)H);
     place("logits", 4 * (size_t)c.vocab);
     place("cand", 8 * (size_t)n_cand);
@@ -1170,6 +1190,8 @@ int build_model(tmq_model* m, const std::vector<Entry>& ents, int max_seq) {
     m->hid[0] = (float*)(B + lay["hid0"]);
     m->hid[1] = (float*)(B + lay["hid1"]);
     m->view = (float*)(B + lay["view"]);
+    m->fin[0] = (float*)(B + lay["fin0"]);
+    m->fin[1] = (float*)(B + lay["fin1"]);
     m->ctxv = (float*)(B + lay["ctx"]);
     m->logits = (float*)(B + lay["logits"]);
     m->cand = (uint64_t*)(B + lay["cand"]);
