@@ -107,6 +107,31 @@ def test_result_over_activation(ctx, oracle, path):
         t.free()
 
 
+# one 16-row workgroup, the last row count of one wave, the first of several,
+# and several workgroups' worth; y before, on and behind the start of x
+@pytest.mark.parametrize("rows", [16, 17, 40, 64, 65, 896])
+def test_fp32_result_over_activation(ctx, oracle, rows):
+    """the same of the FP32 branch, whose 16-row workgroups read x while others store"""
+    import torch
+    import tmq
+    n = 896
+    print(f"[single] fp32 in place {rows}x{n}", flush=True)
+    w = synth.gen_weights(Q5_0, rows, n, 53 + rows)
+    x = synth.gen_x(n, 54)
+    want = oracle.matmul_fp32(Q5_0, w, x, rows, n)
+    t = ctx.upload(Q5_0, rows, n, w)
+    try:
+        for off in (0, 64, -8, n - 4):
+            buf = torch.zeros(3 * n, dtype=torch.float32, device="cuda")
+            buf[64:64 + n] = torch.from_numpy(x)
+            torch.cuda.synchronize()
+            ctx.gemv_dev_path(t, tmq.PATH_FP32, buf.data_ptr() + 256, buf.data_ptr() + 256 + 4 * off)
+            ctx.sync()
+            assert np.array_equal(bits(buf[64 + off:64 + off + rows].cpu().numpy()), bits(want)), off
+    finally:
+        t.free()
+
+
 def chain_of(ctx, torch, shapes, share=None):
     """(chain, xs, x host, y, weights) of (type, rows, cols, activation) rows"""
     import tmq

@@ -440,13 +440,12 @@ TmqWork make_work(const tmq_tensor* t, const uint8_t* act, float* y, int64_t* ac
 // it, a copy in the activation buffer `act` (behind its x_scale).
 int own_x(tmq_ctx* ctx, const tmq_tensor* t, uint8_t* act, const float* x, const float* y, const int64_t* acc,
           size_t acc_per, const float** out) {
-    const uintptr_t x0 = (uintptr_t)x, x1 = x0 + sizeof(float) * (size_t)t->dev.cols;
-    auto over = [&](const void* p, size_t n) { return p && (uintptr_t)p < x1 && x0 < (uintptr_t)p + n; };
+    const size_t xb = sizeof(float) * (size_t)t->dev.cols, rows = (size_t)t->dev.rows;
     *out = x;
-    if (!over(y, sizeof(float) * (size_t)t->dev.rows) && !over(acc, sizeof(int64_t) * acc_per * (size_t)t->dev.rows))
+    if (!tmq_lies_over(x, xb, y, sizeof(float) * rows) && !tmq_lies_over(x, xb, acc, sizeof(int64_t) * acc_per * rows))
         return 0;
     float* c = (float*)(act + 16);
-    HIP_TRY(hipMemcpyAsync(c, x, sizeof(float) * (size_t)t->dev.cols, hipMemcpyDeviceToDevice, ctx->stream));
+    HIP_TRY(hipMemcpyAsync(c, x, xb, hipMemcpyDeviceToDevice, ctx->stream));
     *out = c;
     return 0;
 }
@@ -918,6 +917,13 @@ int tmq_gemv_dev_path(tmq_ctx* ctx, const tmq_tensor* t, int path, const float* 
         if (acc_dev) return tmq_fail(TMQ_ERR_ARG, "the FP32 path has no integer partials (acc_dev must be NULL)");
         w.path = TMQ_WPATH_FP32;
         w.xf = x_dev;
+        // y over x: one wave needs no copy, nor a buffer for it; more rows do
+        if (t->dev.rows > TMQ_F32_ONE_WAVE &&
+            tmq_lies_over(x_dev, sizeof(float) * (size_t)t->dev.cols, y_dev, sizeof(float) * (size_t)t->dev.rows)) {
+            rc = ctx->act.ensure(tmq_act_bytes(t->dev.cols));
+            if (!rc) rc = own_x(ctx, t, (uint8_t*)ctx->act.p, x_dev, y_dev, nullptr, 0, &w.xf);
+            if (rc) return rc;
+        }
         LAUNCH_TRY(tmq_launch_gemv(w, ctx->stream));
         return 0;
     }

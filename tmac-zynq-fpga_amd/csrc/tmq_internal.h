@@ -235,6 +235,10 @@ struct TmqActJobs {
 struct ihipStream_t;
 typedef struct ihipStream_t* hipStream_t;
 int tmq_launch_act_prep(const TmqActJobs& jobs, hipStream_t s);
+// whether the an bytes at a and the bn bytes at b share one (null: none)
+static inline bool tmq_lies_over(const void* a, size_t an, const void* b, size_t bn) {
+    return a && b && (uintptr_t)a < (uintptr_t)b + bn && (uintptr_t)b < (uintptr_t)a + an;
+}
 // n floats (a multiple of 4, 16-byte aligned) from pinned host memory
 int tmq_launch_stage_x(const float* src, float* dst, int n, hipStream_t s);
 int tmq_launch_repack(int type, const uint8_t* src, const TmqTensorDev& t, hipStream_t s);
@@ -263,12 +267,16 @@ int tmq_launch_rowstat(const TmqTensorDev& t, const float* aux_max_abs, float* r
 // A GEMV from a prepared activation (w.act), or, where w.xf is set instead
 // (INT16 and FP32 works, and FPGA works of a tensor that tmq_gemv_takes_x
 // says yes to), from the fp32 activation itself; x_scale goes to *w.xs_out
-// (not FP32).  With w.xf no result may lie over the activation.
+// (not FP32).  With w.xf no result may lie over the activation, but the y of
+// an FP32 work of up to TMQ_F32_ONE_WAVE rows.
 int tmq_launch_gemv(const TmqWork& w, hipStream_t s);
 // FP32 works of up to this many rows run 16 rows a workgroup (the engine's
 // too, but for those that leave argmax candidates), others a lane a row
 #define TMQ_F32_ROWS_MAX 65536
 #define TMQ_F32_ROWS 16
+// of up to this many rows with y over x: all in one wave, a lane a row, which
+// has read the whole activation before it stores
+#define TMQ_F32_ONE_WAVE 64
 bool tmq_gemv_takes_x(const TmqTensorDev& t);
 // before the first of them on a device (current): their kernels' LDS limits
 int tmq_gemv_prepare();

@@ -4244,8 +4244,11 @@ int tmq_launch_gemv(const TmqWork& w, hipStream_t s) {
         } else {
             // above this many rows a lane a row fills the chip (65000 x 896
             // 30 us either way; 151936 x 896 35 us, 69 on f32_rows_kernel;
-            // 32768 x 896 31 against 17)
-            if (w.t.rows > TMQ_F32_ROWS_MAX) {
+            // 32768 x 896 31 against 17); y over x is safe in its one wave
+            // only (the 16-row workgroups read x while others store)
+            const bool in_place = w.t.rows <= TMQ_F32_ONE_WAVE &&
+                                  tmq_lies_over(w.xf, sizeof(float) * (size_t)w.t.cols, w.y, sizeof(float) * (size_t)w.t.rows);
+            if (w.t.rows > TMQ_F32_ROWS_MAX || in_place) {
                 const int g = (w.t.rows_pad / 64 + TMQ_WAVES - 1) / TMQ_WAVES;
                 hipLaunchKernelGGL(f32_gemv_kernel, dim3(g), dim3(64 * TMQ_WAVES), 0, s, w);
                 return (int)hipGetLastError();
