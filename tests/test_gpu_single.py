@@ -51,6 +51,24 @@ def test_fp32_edges(ctx, oracle, qt, rows, cols):
     assert np.array_equal(bits(y), bits(oracle.matmul_fp32(qt, w, x, rows, cols)))
 
 
+# the last row count of the 16-row workgroups and the first of a lane a row, by
+# type: 32, 48 and 60 rows a column, and the narrowest of them
+@pytest.mark.parametrize("qt,cols", [(F32, 128), (F32, 160), (F16, 96), (F16, 128), (Q8_0, 160), (Q5_0, 128), (Q4_K, 256)])
+def test_fp32_bounds(ctx, oracle, qt, cols):
+    import tmq
+    per = {F32: 32, F16: 48, Q8_0: 48}.get(qt, 60)
+    x = synth.gen_x(cols, 63 + cols)
+    for rows in (per * cols, per * cols + 1):
+        print(f"[single] fp32 type={qt} {rows}x{cols}", flush=True)
+        w = synth.gen_weights(qt, rows, cols, 64 + cols)
+        t = ctx.upload(qt, rows, cols, w)
+        try:
+            y = ctx.matmul_path(t, x, tmq.PATH_FP32)
+        finally:
+            t.free()
+        assert np.array_equal(bits(y), bits(oracle.matmul_fp32(qt, w, x, rows, cols))), rows
+
+
 # the 16-row MFMA GEMVs: 1 and 3 blocks of a step's 4, 8 waves' worth (32) and
 # one step more, the widest; one and two super-blocks, more than 8 waves', the
 # bounds of the x registers (1024, 5120); rows 1, 16k, 16k + 1, and the first

@@ -4232,6 +4232,23 @@ bool tmq_gemv_takes_x(const TmqTensorDev& t) {
     if (f == kQ8_0) return t.cols <= kQ8WideCols ? (int64_t)t.rows * t.cols <= 1 << 27 : t.rows <= 49152;
     return (f == kQ5_0M || f == kQ4_KM || f == kQ6_KM) && t.rows <= 16384 && (int64_t)t.rows * t.cols <= 1 << 25;
 }
+// Rows up to which an FP32 work runs 16 rows a workgroup.  Above, a lane a row
+// fills the chip; how soon depends on the columns, of which a 16-row
+// workgroup's cost is only half, and on the bytes of an element.  us, 16 rows
+// a workgroup against a lane a row: Q5_0 12288 x 128 3.8 against 4.8, 32768 x
+// 256 8.4 / 7.8, 40000 x 640 16.2 / 17.3, 49152 x 768 20.7 / 19.9, 65536 x
+// 1280 39 / 43, 151936 x 896 69 / 35; Q6_K 32768 x 512 13.5 / 17.5; Q8_0
+// 12288 x 256 4.0 / 6.8, 36864 x 512 12.6 / 11.8, 49152 x 1024 25.7 / 30.8,
+// 65536 x 1024 33.8 / 30.4; F16 24576 x 512 9.1 / 10.4, 40000 x 512 15.9 /
+// 15.1; F32 12288 x 384 5.1 / 6.6, 16384 x 384 7.1 / 6.6, 24576 x 2048 33.6 /
+// 38.8, 49152 x 2048 75 / 62.  Fewer columns than one producer's 128 leave
+// either way at the launch's own time (3.4 against 3.7).
+static int f32_rows_max(const TmqTensorDev& t) {
+    const bool f32 = t.type == kF32;
+    if (t.cols < (f32 ? 160 : 128)) return 0;
+    const int per = f32 ? 32 : t.type == kF16 || t.type == kQ8_0 ? 48 : 60;
+    return (int)std::min<int64_t>(f32 ? 24576 : TMQ_F32_ROWS_MAX, (int64_t)per * t.cols);
+}
 int tmq_launch_gemv(const TmqWork& w, hipStream_t s) {
     if (w.ngroups <= 0) return 0;
     if (w.path != TMQ_WPATH_FPGA) {
@@ -4242,13 +4259,11 @@ int tmq_launch_gemv(const TmqWork& w, hipStream_t s) {
             const int nw = tiles_waves(w.t.cols);
             hipLaunchKernelGGL(i16_gemv_kernel, dim3(w.t.rows_pad / kTileRows), dim3(64 * nw), tiles_lds(w.t.cols, nw), s, w);
         } else {
-            // above this many rows a lane a row fills the chip (65000 x 896
-            // 30 us either way; 151936 x 896 35 us, 69 on f32_rows_kernel;
-            // 32768 x 896 31 against 17); y over x is safe in its one wave
-            // only (the 16-row workgroups read x while others store)
+            // y over x is safe in the one wave of a lane a row only (the
+            // 16-row workgroups read x while others store)
             const bool in_place = w.t.rows <= TMQ_F32_ONE_WAVE &&
                                   tmq_lies_over(w.xf, sizeof(float) * (size_t)w.t.cols, w.y, sizeof(float) * (size_t)w.t.rows);
-            if (w.t.rows > TMQ_F32_ROWS_MAX || in_place) {
+            if (w.t.rows > f32_rows_max(w.t) || in_place) {
                 const int g = (w.t.rows_pad / 64 + TMQ_WAVES - 1) / TMQ_WAVES;
                 hipLaunchKernelGGL(f32_gemv_kernel, dim3(g), dim3(64 * TMQ_WAVES), 0, s, w);
                 return (int)hipGetLastError();
