@@ -34,6 +34,26 @@ def test_int16_edges(ctx, oracle, qt, rows, cols):
     assert np.array_equal(bits(y), bits(ye))
 
 
+# the last row count of the 8-row workgroups and the first of a lane a row:
+# 57344 up to 128 columns, 768 a column above
+@pytest.mark.parametrize("rows,cols", [(57344, 32), (57345, 96), (57345, 128), (122880, 160), (122881, 160)])
+def test_int16_bounds(ctx, oracle, rows, cols):
+    import tmq
+    print(f"[single] int16 {rows}x{cols}", flush=True)
+    w = synth.gen_weights(Q5_0, rows, cols, 43 + cols)
+    x = synth.gen_x(cols, 44 + cols)
+    t = ctx.upload(Q5_0, rows, cols, w)
+    try:
+        acc, xs = ctx.partials_int16(t, x)
+        y = ctx.matmul_path(t, x, tmq.PATH_INT16)
+    finally:
+        t.free()
+    ye, te, _ = oracle.matmul_int16(Q5_0, w, x, rows, cols)
+    assert xs == oracle.quantize_act(x)[1]
+    assert np.array_equal(acc, te)
+    assert np.array_equal(bits(y), bits(ye))
+
+
 # 384 columns a batch: one block, one batch exactly, one block more, two
 # batches and a half; rows 1, 16k, 16k + 1, and past the lane-a-row bound
 @pytest.mark.parametrize("qt,rows,cols", [(F32, 1, 32), (Q8_0, 16, 384), (Q5_0, 17, 416), (F16, 40, 960), (Q4_K, 5, 1024),

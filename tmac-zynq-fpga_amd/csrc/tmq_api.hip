@@ -450,6 +450,17 @@ int own_x(tmq_ctx* ctx, const tmq_tensor* t, uint8_t* act, const float* x, const
     return 0;
 }
 
+// x quantised into `act` by a launch of its own
+int prep_x(tmq_ctx* ctx, const tmq_tensor* t, uint8_t* act, const float* x) {
+    TmqActJobs jobs{};
+    jobs.count = 1;
+    jobs.j[0].x = x;
+    jobs.j[0].act = act;
+    jobs.j[0].n = t->dev.cols;
+    LAUNCH_TRY(tmq_launch_act_prep(jobs, ctx->stream));
+    return 0;
+}
+
 // A tensor's own kernel on a device activation; `act` (tmq_act_bytes) gets
 // x_scale and, where the kernel reads one, the prepared activation.
 int gemv_fpga(tmq_ctx* ctx, const tmq_tensor* t, uint8_t* act, const float* x, float* y, int64_t* acc) {
@@ -459,12 +470,8 @@ int gemv_fpga(tmq_ctx* ctx, const tmq_tensor* t, uint8_t* act, const float* x, f
         if (rc) return rc;
         w.xs_out = (float*)act;
     } else {
-        TmqActJobs jobs{};
-        jobs.count = 1;
-        jobs.j[0].x = x;
-        jobs.j[0].act = act;
-        jobs.j[0].n = t->dev.cols;
-        LAUNCH_TRY(tmq_launch_act_prep(jobs, ctx->stream));
+        const int rc = prep_x(ctx, t, act, x);
+        if (rc) return rc;
     }
     LAUNCH_TRY(tmq_launch_gemv(w, ctx->stream));
     return 0;
@@ -927,16 +934,21 @@ int tmq_gemv_dev_path(tmq_ctx* ctx, const tmq_tensor* t, int path, const float* 
         LAUNCH_TRY(tmq_launch_gemv(w, ctx->stream));
         return 0;
     }
-    // INT16: weights quantised once per tensor; the kernel quantises the
-    // activation and leaves x_scale at the start of the context's buffer
+    // INT16: weights quantised once per tensor; the kernel (or a launch in
+    // front of it) quantises the activation and leaves x_scale at the start of
+    // the context's buffer
     rc = tmq_rt_prepare_int16(ctx, const_cast<tmq_tensor*>(t));
     if (!rc) rc = ctx->act.ensure(tmq_act_bytes(t->dev.cols));
     if (rc) return rc;
-    w = make_work(t, nullptr, y_dev, acc_dev);
+    w = make_work(t, (const uint8_t*)ctx->act.p, y_dev, acc_dev);
     w.path = TMQ_WPATH_INT16;
-    rc = own_x(ctx, t, (uint8_t*)ctx->act.p, x_dev, y_dev, acc_dev, (size_t)((t->dev.cols + 63) / 64), &w.xf);
+    if (tmq_i16_takes_x(t->dev)) {
+        rc = own_x(ctx, t, (uint8_t*)ctx->act.p, x_dev, y_dev, acc_dev, (size_t)((t->dev.cols + 63) / 64), &w.xf);
+        w.xs_out = (float*)ctx->act.p;
+    } else {
+        rc = prep_x(ctx, t, (uint8_t*)ctx->act.p, x_dev);
+    }
     if (rc) return rc;
-    w.xs_out = (float*)ctx->act.p;
     LAUNCH_TRY(tmq_launch_gemv(w, ctx->stream));
     return 0;
 }

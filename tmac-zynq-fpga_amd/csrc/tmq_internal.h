@@ -265,8 +265,8 @@ static inline int tmq_ifit_subs(int type) { return type == 6 ? 1 : type == 12 ? 
 int tmq_launch_rowstat(const TmqTensorDev& t, const float* aux_max_abs, float* row_inv,
                        float* row_scale, int* bad_flag, hipStream_t s);
 // A GEMV from a prepared activation (w.act), or, where w.xf is set instead
-// (INT16 and FP32 works, and FPGA works of a tensor that tmq_gemv_takes_x
-// says yes to), from the fp32 activation itself; x_scale goes to *w.xs_out
+// (FP32 works, and INT16 and FPGA works of a tensor that tmq_i16_takes_x or
+// tmq_gemv_takes_x says yes to), from the fp32 activation itself; x_scale goes to *w.xs_out
 // (not FP32).  With w.xf no result may lie over the activation, but the y of
 // an FP32 work of up to TMQ_F32_ONE_WAVE rows.
 int tmq_launch_gemv(const TmqWork& w, hipStream_t s);
@@ -279,6 +279,7 @@ int tmq_launch_gemv(const TmqWork& w, hipStream_t s);
 // has read the whole activation before it stores
 #define TMQ_F32_ONE_WAVE 64
 bool tmq_gemv_takes_x(const TmqTensorDev& t);
+bool tmq_i16_takes_x(const TmqTensorDev& t);  // the same of INT16 works
 // before the first of them on a device (current): their kernels' LDS limits
 int tmq_gemv_prepare();
 // One workgroup of a chain launch: row group `group` of works[work] over

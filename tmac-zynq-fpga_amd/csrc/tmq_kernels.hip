@@ -2471,6 +2471,29 @@ __device__ __forceinline__ int64_t i16_tile(const TmqTensorDev& t, const AT& A, 
     return (int64_t)sh * 256 + sl;
 }
 
+// matmul_fpga_int16 (sim/tmac_gguf.cpp:887-940) of very many short rows
+// (tmq_i16_takes_x): 4 waves of 64 rows, a lane a row, walk the 64-column tiles
+// in order from a prepared activation.  The 8-row workgroups' fixed cost is 8
+// times as many workgroups' there: 151936 x 32 13.1 us against 6.6 with the
+// quantisation's launch, 65536 x 64 7.7 / 7.2, 120000 x 128 12.2 / 10.9.
+__global__ __launch_bounds__(64 * TMQ_WAVES) void i16_lanes_kernel(TmqWork w) {
+    const TmqTensorDev& t = w.t;
+    const int lane = threadIdx.x & 63, wave = wave_id();
+    const int r0 = (blockIdx.x * TMQ_WAVES + wave) * 64;
+    if (r0 >= t.rows_pad) return;
+    const int r = r0 + lane;
+    const double rs = (double)t.rs16[r];
+    const Act A = act_view(w.act);
+    const int nt = (t.cols + 63) / 64;
+    float y = 0.0f;
+    for (int tt = 0; tt < nt; tt++) {
+        const int64_t P = i16_tile(t, A, r, tt);
+        if (w.acc && r < t.rows) w.acc[(size_t)r * nt + tt] = P;
+        y = (float)((double)y + ((double)P * (double)A.xs) * rs);
+    }
+    if (w.y && r < t.rows) store_y(w, r, y);
+}
+
 // matmul_fpga_int16 (sim/tmac_gguf.cpp:887-940): group_tiles on the rounded
 // weights.  One wave walking the tiles of 64 rows behind a quantisation
 // launch left 14 waves for 896 rows.  A call, launches included: 896 x 4864
@@ -4232,6 +4255,14 @@ bool tmq_gemv_takes_x(const TmqTensorDev& t) {
     if (f == kQ8_0) return t.cols <= kQ8WideCols ? (int64_t)t.rows * t.cols <= 1 << 27 : t.rows <= 49152;
     return (f == kQ5_0M || f == kQ4_KM || f == kQ6_KM) && t.rows <= 16384 && (int64_t)t.rows * t.cols <= 1 << 25;
 }
+// One launch of 8-row workgroups, but for very many short rows, us against the
+// quantisation and i16_lanes_kernel: 49152 x 32 6.2 / 6.5, 65536 x 32 7.1 /
+// 6.6, 65536 x 96 7.8 / 8.0, 90000 x 128 9.7 / 8.7; 120000 x 160 12.6 / 12.8,
+// 151936 x 192 15.4 / 15.4, 151936 x 256 16.0 / 18.6, 400000 x 256 36.6 / 33.7,
+// 400000 x 512 86 / 73.
+bool tmq_i16_takes_x(const TmqTensorDev& t) {
+    return t.rows <= (t.cols <= 128 ? 57344 : (int64_t)768 * t.cols);
+}
 // Rows up to which an FP32 work runs 16 rows a workgroup.  Above, a lane a row
 // fills the chip; how soon depends on the columns, of which a 16-row
 // workgroup's cost is only half, and on the bytes of an element.  us, 16 rows
@@ -4252,10 +4283,17 @@ static int f32_rows_max(const TmqTensorDev& t) {
 int tmq_launch_gemv(const TmqWork& w, hipStream_t s) {
     if (w.ngroups <= 0) return 0;
     if (w.path != TMQ_WPATH_FPGA) {
-        // INT16 / FP32 paths, from the fp32 activation
+        // INT16 / FP32 paths, from the fp32 activation but for many short rows
+        if (w.path == TMQ_WPATH_INT16 && !w.xf) {
+            if (!w.t.pw || !w.t.rs16 || !w.act) return (int)hipErrorInvalidValue;
+            const int g = (w.t.rows_pad / 64 + TMQ_WAVES - 1) / TMQ_WAVES;
+            hipLaunchKernelGGL(i16_lanes_kernel, dim3(g), dim3(64 * TMQ_WAVES), 0, s, w);
+            return (int)hipGetLastError();
+        }
         if (!w.xf) return (int)hipErrorInvalidValue;
         if (w.path == TMQ_WPATH_INT16) {
             if (!w.t.pw || !w.t.rs16 || !w.xs_out) return (int)hipErrorInvalidValue;
+            if (!tmq_i16_takes_x(w.t)) return (int)hipErrorInvalidValue;
             const int nw = tiles_waves(w.t.cols);
             hipLaunchKernelGGL(i16_gemv_kernel, dim3(w.t.rows_pad / kTileRows), dim3(64 * nw), tiles_lds(w.t.cols, nw), s, w);
         } else {
