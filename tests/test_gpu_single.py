@@ -96,7 +96,8 @@ def test_fp32_bounds(ctx, oracle, qt, cols):
 @pytest.mark.parametrize("qt,rows,cols", [
     (Q5_0, 1, 32), (Q5_0, 17, 96), (Q5_0, 48, 1024), (Q5_0, 65, 1056), (Q5_0, 16, 8192), (Q5_0, 16385, 96),
     (Q4_K, 1, 256), (Q4_K, 33, 1024), (Q4_K, 64, 1280), (Q4_K, 15, 8192),
-    (Q6_K, 1, 256), (Q6_K, 31, 512), (Q6_K, 80, 5120), (Q6_K, 17, 5376), (Q6_K, 4097, 8192)])
+    (Q6_K, 1, 256), (Q6_K, 31, 512), (Q6_K, 80, 5120), (Q6_K, 17, 5376), (Q6_K, 4097, 8192),
+    (Q6_K, 12288, 256), (Q6_K, 12289, 256), (Q4_K, 12289, 256), (Q4_K, 12289, 1280)])
 @pytest.mark.parametrize("force", [0, 1])
 def test_fpga_edges(ctx, oracle, monkeypatch, qt, rows, cols, force):
     if force and rows > 100:
@@ -250,7 +251,7 @@ def test_chain_shared_result(ctx, oracle):
 
 # both one-launch Q8_0 kernels around their bound, half tiles, batches
 @pytest.mark.parametrize("rows,cols", [(1, 32), (9, 544), (7, 8192), (33, 9248), (8192, 96), (8193, 96), (8257, 544),
-                                       (8193, 4096), (8200, 4128)])
+                                       (8193, 4096), (8200, 4128), (196608, 32), (196609, 32)])
 def test_q8_edges(ctx, oracle, rows, cols):
     print(f"[single] q8_0 {rows}x{cols}", flush=True)
     w = synth.gen_weights(Q8_0, rows, cols, 31 + rows)

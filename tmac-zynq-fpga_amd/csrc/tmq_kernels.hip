@@ -4244,16 +4244,24 @@ constexpr int kTilesMaxRows = 8192;
 // the time grows with the weights (0.35 ns a row of 896 Q5_0, 0.62 of 1024
 // and 2.5 of 4096 Q6_K columns) where the two launches' is flat (10 us at
 // 896 columns, 12 at 1024, 20 at 4096, 32 at 8192).
-// Q5_0 16000 x 896 8.5 against 10.0 us, 65000 x 896 25.6 against 14.2;
-// Q6_K 20000 x 1024 14.7 against 12.1, 5000 x 4096 11.8 against 19.6.
+// It rises by steps, a round of two workgroups a CU (8192 rows) and its
+// halves: the K-quants' step at 12289 rows is the first above the two
+// launches, but for Q4_K's of up to 1024 columns.  us, one launch / two, at
+// 12288 and 16384 rows: Q5_0 x 1024 6.6 / 9.8 and 8.2 / 9.8, x 2048 9.3 / 12.9
+// and 11.6 / 13.1; Q4_K x 1024 7.4 / 8.8 and 8.9 / 9.4, x 2048 9.6 / 11.8 and
+// 12.1 / 11.8; Q6_K x 1024 8.5 / 10.0 and 10.8 / 10.1, x 2048 11.6 / 12.9 and
+// 14.9 / 13.0; at 8192 rows x 4096 Q5_0 10.5 / 19.5, Q4_K 9.9 / 16.7, Q6_K
+// 11.4 / 19.4, at 4096 x 8192 11.0 / 33.9, 10.1 / 28.4, 11.2 / 33.3.
 bool tmq_gemv_takes_x(const TmqTensorDev& t) {
     const int f = tmq_kernel_fmt(t);
     // Q8_0: one launch up to 128 M weights (151936 x 896 28.4 us on the wide
     // kernel, 28.0 on two launches; 100000 x 896 18.6 against 24.9), and
     // where only 8-row workgroups take the width, up to 49152 rows (32000 x
-    // 4096 46 against 79)
-    if (f == kQ8_0) return t.cols <= kQ8WideCols ? (int64_t)t.rows * t.cols <= 1 << 27 : t.rows <= 49152;
-    return (f == kQ5_0M || f == kQ4_KM || f == kQ6_KM) && t.rows <= 16384 && (int64_t)t.rows * t.cols <= 1 << 25;
+    // 4096 46 against 79); very many short rows are workgroups of one tile
+    // each (200000 x 32 6.2 against 6.8, 300000 x 32 8.1 against 7.1)
+    if (f == kQ8_0) return t.rows <= 196608 && (t.cols <= kQ8WideCols ? (int64_t)t.rows * t.cols <= 1 << 27 : t.rows <= 49152);
+    const int rows = f == kQ5_0M || (f == kQ4_KM && t.cols <= 1024) ? 16384 : f == kQ4_KM || f == kQ6_KM ? 12288 : 0;
+    return t.rows <= rows && (int64_t)t.rows * t.cols <= 1 << 25;
 }
 // One launch of 8-row workgroups, but for very many short rows, us against the
 // quantisation and i16_lanes_kernel: 49152 x 32 6.2 / 6.5, 65536 x 32 7.1 /
