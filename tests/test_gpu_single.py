@@ -220,6 +220,30 @@ def test_chain_one_launch(ctx, oracle):
     ch.free()
 
 
+# Q6_K of 6144 and of 8192 columns (two and one workgroup a CU) on either side
+# of their bounds: 32 and 33, 16 and 17 tensors of 256 rows on 256 CUs
+@pytest.mark.parametrize("cols,n", [(6144, 32), (6144, 33), (8192, 16), (8192, 17)])
+def test_chain_one_bounds(ctx, oracle, cols, n):
+    import torch
+    import tmq
+    rows = 256
+    print(f"[single] chain of {n} q6_k {rows}x{cols}", flush=True)
+    x = synth.gen_x(cols, 95)
+    w = synth.gen_weights(Q6_K, rows, cols, 96)
+    want = oracle.matmul(Q6_K, w, x, rows, cols)
+    t = ctx.upload(Q6_K, rows, cols, w)
+    xd = torch.from_numpy(x).cuda()
+    ys = [torch.zeros(rows, dtype=torch.float32, device="cuda") for _ in range(n)]
+    torch.cuda.synchronize()
+    ch = tmq.Chain(ctx, [(t, xd.data_ptr(), y.data_ptr(), None, 8 * (cols // 256), 32, cols // 256) for y in ys])
+    ch.run()
+    ctx.sync()
+    for i, y in enumerate(ys):
+        assert np.array_equal(bits(y.cpu().numpy()), bits(want)), i
+    ch.free()
+    t.free()
+
+
 def test_chain_result_over_activation(ctx, oracle):
     """every activation is quantised before any result is stored"""
     import torch

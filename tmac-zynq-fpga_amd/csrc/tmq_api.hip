@@ -581,13 +581,20 @@ void plan_segments(std::vector<TmqWork>& works, std::vector<TmqGroupRef>& gmap, 
 
 // Whether the chain's runs take one launch, and its group map (appended).
 // Every workgroup of it quantises its activation again, so the line is drawn
-// by their number: up to two a CU for each launch of a format it replaces.
+// by their number: as many as are resident at once (two a CU; one where the
+// widest K-quant rows fill the LDS) for each launch of a format it replaces.
 // us, one launch against the quantisation and the formats' launches: a layer
 // of Q5_0, Q8_0 and Q6_K products (330 workgroups) 10.6 against 25.5, three
 // 20.0 against 29.5, five 27.3 against 32.8; attn_q, gate and up in Q5_0
 // (184) 6.6 against 10.2, three times 11.6 against 11.1; 896 x 4864 Q6_K
 // (56) 9.2 against 11.8, eight 15.3 against 17.3, Q4_K 12.9 against 15.7;
-// 4864 x 896 Q8_0 (76) 6.5 against 10.4, eight 12.3 against 22.5.
+// 4864 x 896 Q8_0 (76) 6.5 against 10.4, eight 12.3 against 22.5; 896 x 8192
+// Q6_K, one workgroup a CU: four (224) 13.0 against 18.1, five (280) 23.7
+// against 20.1, nine 26.6 against 23.5.  A Q8_0 workgroup counts half, for
+// what it costs: 64 rows, where its format's own launch is a wave a row too;
+// up to twice the resident number are still ahead, 72 of 896 x 896 (1008
+// workgroups) 15.2 against 22.1, 72 of 896 x 4096 50 against 84, four of
+// 16384 x 256 (1024) 9.4 against 10.5.
 void plan_one(tmq_chain* ch, std::vector<TmqGroupRef>& gmap, int ncu) {
     int64_t groups = 0;
     size_t lds = 0;
@@ -604,7 +611,7 @@ void plan_one(tmq_chain* ch, std::vector<TmqGroupRef>& gmap, int ncu) {
     for (const TmqWork& w : ch->works) {
         if (!tmq_chain_one_rows(w.t)) return;
         const int64_t n = w.t.rows_pad / tmq_chain_one_rows(w.t);
-        groups += w.t.type == TMQ_TYPE_Q8_0 ? (n + 1) / 2 : n;  // (four resident where the others are two)
+        groups += w.t.type == TMQ_TYPE_Q8_0 ? (n + 1) / 2 : n;
         lds = std::max(lds, tmq_chain_one_lds(w.t));
         // a result over an activation: all of them are quantised first
         for (int a = 0; a < ch->jobs.count; a++) {
@@ -614,7 +621,7 @@ void plan_one(tmq_chain* ch, std::vector<TmqGroupRef>& gmap, int ncu) {
             if (over(w.y, sizeof(float) * (size_t)w.t.rows) || over(w.acc, sizeof(int64_t) * per * (size_t)w.t.rows)) return;
         }
     }
-    if (groups > 2 * (int64_t)ncu * (int64_t)ch->segs.size()) return;
+    if (groups > tmq_chain_one_resident(lds) * (int64_t)ncu * (int64_t)ch->segs.size()) return;
     ch->one_off = (int)gmap.size();
     ch->one_lds = lds;
     for (size_t i = 0; i < ch->works.size(); i++) {

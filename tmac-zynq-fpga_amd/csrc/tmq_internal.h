@@ -307,6 +307,7 @@ int tmq_launch_chain(int fmt, int clamp, int max_cols, const TmqWork* works_dev,
 // tmq_chain_one_lds of them.  No result may lie over an activation.
 int tmq_chain_one_rows(const TmqTensorDev& t);
 size_t tmq_chain_one_lds(const TmqTensorDev& t);
+int tmq_chain_one_resident(size_t lds);  // workgroups of it a CU holds at once
 int tmq_launch_chain_one(const TmqActJobs& jobs, const TmqWork* works_dev, const TmqGroupRef* groups_dev, int ngroups,
                          size_t lds, hipStream_t s);
 // widest Q8_0 rows whose chain groups split into quarters (the quarters'

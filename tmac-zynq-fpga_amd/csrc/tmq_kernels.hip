@@ -2233,7 +2233,8 @@ __global__ __launch_bounds__(1024) void one_q8_kernel(TmqWork w) {
 // (act_prep_kernel's, for the callers that launch the chain again without
 // quantising), then the descriptors' workgroups (one_rows), which quantise
 // for themselves.  Descriptor -> works[], workgroup -> (descriptor, row
-// group) through groups[].  Held to 128 registers: two workgroups a CU.
+// group) through groups[].  Held to 128 registers, two workgroups a CU, at
+// the price of seven spilled around two formats' block loops (24 B a lane).
 __device__ void act_prep(const TmqActJob& J, float* red);
 __host__ __device__ inline int one_rows(const TmqTensorDev& t) {
     // Q5_0 of many rows: 64 a workgroup, four times fewer quantisations
@@ -4399,6 +4400,12 @@ size_t tmq_chain_one_lds(const TmqTensorDev& t) {
     case kQ6_KM: return one_lds<kQ6_KM>(nbx);
     default: return q8_wide_lds(t.cols);
     }
+}
+int tmq_chain_one_resident(size_t lds) {
+    // two by its registers; the LDS of a CU is 160 KiB, given out in steps
+    // (512: the kernel's own arrays)
+    const size_t each = (lds + 512 + 2047) & ~(size_t)2047;
+    return 2 * each <= 160 * 1024 ? 2 : 1;
 }
 int tmq_launch_chain_one(const TmqActJobs& jobs, const TmqWork* works_dev, const TmqGroupRef* groups_dev, int ngroups,
                          size_t lds, hipStream_t s) {
