@@ -351,8 +351,10 @@ def test_chain_split_tail_q8(ctx, oracle, monkeypatch):
     each, the last one half empty) and one 130x896 tensor (1 group): 81
     groups leave a last round of 81 on 256 CUs, which the chain runs as one
     workgroup per 64-row quarter, the four waves splitting the row's tiles.
-    Three runs: per-tile int64 sums and fp32 outputs bit-exact with the
-    oracle, the same as the unsplit chain (TMQ_NOSPLIT=1)."""
+    Three runs of the format's own launch (prepare + launch), then three of
+    the run that a chain this small takes, one launch of 64-row workgroups:
+    per-tile int64 sums and fp32 outputs bit-exact with the oracle, the same
+    as the unsplit chain (TMQ_NOSPLIT=1)."""
     torch = pytest.importorskip("torch")
     dev = torch.device("cuda:0")
     cols = 896
@@ -378,11 +380,13 @@ def test_chain_split_tail_q8(ctx, oracle, monkeypatch):
         monkeypatch.setenv("TMQ_NOSPLIT", "1" if nosplit else "0")
         print(f"[chain] Q8_0 split tail, nosplit {nosplit}", flush=True)
         ch = ctx.chain(descs)
-        for run in range(3):
+        ch.prepare()
+        for run, go in enumerate([ch.launch] * 3 + [ch.run] * 3):
             for y, a in zip(ys, accs):
                 y.zero_()
                 a.zero_()
-            ch.run()
+            torch.cuda.synchronize()
+            go()
             ctx.sync()
             for i, (y, a, (pe, ye)) in enumerate(zip(ys, accs, exp)):
                 got = a.cpu().numpy()
