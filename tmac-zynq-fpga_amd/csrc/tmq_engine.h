@@ -26,7 +26,7 @@ struct TmqAttnArgs {
     float* sc;               // [n_heads][max_pos]
     uint32_t* cnt;           // [n_heads], zero between launches
     int32_t n_split;         // set by the launch
-    int32_t pad_;
+    int32_t spec_miss;       // nonzero: the exp sum's segments all re-run (testing)
 };
 
 int tmq_launch_attn(const TmqAttnArgs& a, hipStream_t s);

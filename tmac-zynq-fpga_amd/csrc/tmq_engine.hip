@@ -104,7 +104,7 @@ __device__ __forceinline__ void attn_long(const TmqAttnArgs& a, float* lds, cons
         if (p < n4) ex[p] = p <= pos ? tmq_math::tmq_expf_tab(sv[k] - mx, Exp2TabLds{tab}) : 0.0f;
     }
     __syncthreads();
-    const float es = seq_sum_spec<8>(ex, n4, prod, (int*)(prod + 512), 0);
+    const float es = seq_sum_spec<8>(ex, n4, prod, (int*)(prod + 512), a.spec_miss);
     if (tid == 0) s_stat[0] = tmq_math::tmq_logf_tab(es, LogfTabLds{ltab}) + mx;
     __syncthreads();
     const float ls = s_stat[0];

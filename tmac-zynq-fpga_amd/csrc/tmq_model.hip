@@ -185,7 +185,7 @@ struct tmq_model {
     // tmq_model_profile: an event before and after every launch
     std::vector<std::pair<const char*, hipEvent_t>>* prof = nullptr;
     int prefill_chunk = 512;  // 0: prompts run one token at a time
-    int spec_miss = 0;        // TMQ_SPEC_MISS=1: every RMSNorm sum segment re-runs (testing)
+    int spec_miss = 0;        // TMQ_SPEC_MISS=1: every speculated sum segment re-runs (testing)
     const char* prefill_off = nullptr;  // why the model cannot use the batched prefill
     Prefill pf;
 };
@@ -290,6 +290,7 @@ int launch_layers(tmq_model* m, bool dump, float* cap = nullptr) {
         aa.max_pos = c.max_seq;
         aa.sc = m->attn_sc;
         aa.cnt = m->attn_cnt;
+        aa.spec_miss = m->spec_miss;
         PROF("rope+attention", LAUNCH_TRY(tmq_launch_attn(aa, s)));
         if (cap) HIP_TRY(hipMemcpyAsync(cap + l * per + H, m->ctxv, sizeof(float) * H, hipMemcpyDeviceToDevice, s));
         PROF("attn_output", rc = launch_gemv_fin(m, L.o_l, L.dout, 0));
