@@ -55,7 +55,7 @@ def test_int16_bounds(ctx, oracle, rows, cols):
 
 
 # 384 columns a batch: one block, one batch exactly, one block more, two
-# batches and a half; rows 1, 16k, 16k + 1, and past the lane-a-row bound
+# batches and a half; rows 1, 16k, 16k + 1; very many of a lane a row
 @pytest.mark.parametrize("qt,rows,cols", [(F32, 1, 32), (Q8_0, 16, 384), (Q5_0, 17, 416), (F16, 40, 960), (Q4_K, 5, 1024),
                                           (Q6_K, 33, 4864), (Q5_0, 65536, 32), (Q5_0, 65537, 64)])
 def test_fp32_edges(ctx, oracle, qt, rows, cols):

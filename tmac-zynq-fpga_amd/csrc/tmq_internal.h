@@ -270,10 +270,8 @@ int tmq_launch_rowstat(const TmqTensorDev& t, const float* aux_max_abs, float* r
 // (not FP32).  With w.xf no result may lie over the activation, but the y of
 // an FP32 work of up to TMQ_F32_ONE_WAVE rows.
 int tmq_launch_gemv(const TmqWork& w, hipStream_t s);
-// FP32 works of up to this many rows (fewer where the row is short:
-// f32_rows_max) run 16 rows a workgroup (the engine's too, but for those that
-// leave argmax candidates), others a lane a row
-#define TMQ_F32_ROWS_MAX 65536
+// rows of a workgroup of an FP32 work (above f32_rows_max rows, and where the
+// engine's leave argmax candidates, a lane takes a row instead)
 #define TMQ_F32_ROWS 16
 // of up to this many rows with y over x: all in one wave, a lane a row, which
 // has read the whole activation before it stores

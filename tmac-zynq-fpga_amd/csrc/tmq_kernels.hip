@@ -2131,8 +2131,8 @@ __global__ __launch_bounds__(64 * kOneWaves) void one_kernel(TmqWork w) {
 }
 // Q8_0 tensors of many rows: 64 rows a workgroup, one a lane, the 64-column
 // tiles over its four waves (x from LDS, the same address in every lane),
-// the next tile's weights on the way while one is multiplied.  2374
-// rows x 896, a call: 16000 21.5 us (two launches of 256-row workgroups, a
+// the next tile's weights on the way while one is multiplied.  Rows
+// x 896, a call: 16000 21.5 us (two launches of 256-row workgroups, a
 // wave a lane's whole row) -> 5.8 (group_tiles 8.1), 65536 22.9 -> 12.9.
 constexpr int kQ8WideCols = 4096;  // (48 KiB of LDS)
 __host__ __device__ constexpr int q8_wide_lds(int cols) { return ((cols + 63) / 64) * (256 + 512); }
@@ -2162,7 +2162,7 @@ __device__ __forceinline__ void group_q8_wide(const TmqWork& w, int g) {
     float m = 0.0f;
 #pragma unroll
     for (int k = 0; k < kXR; k++) m = fmaxf(m, fabsf(xv[k]));
-    for (int j = tid + 64 * NW * kXR; j < n; j += 256) m = fmaxf(m, fabsf(w.xf[j]));
+    for (int j = tid + 64 * NW * kXR; j < n; j += 64 * NW) m = fmaxf(m, fabsf(w.xf[j]));
     m = tmq_wave_max(m);
     if (lane == 0) red[wave] = m;
     __syncthreads();
@@ -3207,13 +3207,11 @@ __device__ __forceinline__ void eng_group_i16(const TmqEngAct& a, const EngLds& 
     if (w.cand) wave_cand(w, r, y, grp);
 }
 
-// FP32 path in the engine (the loop of :488-492): each wave owns 64 rows,
-// one lane per row, and sums read_tensor(r, j) * o_j in column order from
-// the launch's fp32 activation o = L.x * red[1] (the rms_norm output
-// fl(fl(x*w)*scale), :447-453, or the input itself).  The rows are final
-// values (TmqDeferred.val); the logits also leave argmax candidates.
-// The FP32 loop of a launch's works (no candidates): 16 rows a workgroup
-// (f32_rows), from the activation the prologue left in LDS.
+// FP32 path in the engine (the loop of :488-492): sums read_tensor(r, j) * o_j
+// in column order from the launch's fp32 activation o = L.x * red[1] (the
+// rms_norm output fl(fl(x*w)*scale), :447-453, or the input itself), which the
+// prologue left in LDS.  The rows are final values (TmqDeferred.val).  The
+// layers' works: 16 rows a workgroup (f32_rows).
 template <int NW, bool MULTI>
 __device__ __forceinline__ void eng_group_f32_rows(const TmqEngAct& a, const EngLds& L, const TmqWork& w, int g) {
     static_assert(NW == 1 + kF32Prod, "f32_rows' waves");
@@ -3231,14 +3229,16 @@ __device__ __forceinline__ void eng_group_f32_rows(const TmqEngAct& a, const Eng
     }
 }
 
-template <int NW, bool MULTI>
+// The logits: each wave owns 64 rows, a lane a row, and leaves an argmax
+// candidate.
+template <int NW>
 __device__ __forceinline__ void eng_group_f32(const TmqEngAct& a, const EngLds& L, const TmqWork& w, int g) {
     const TmqTensorDev& t = w.t;
     const int lane = threadIdx.x & 63, wave = wave_id();
     const int grp = g * NW + wave, r0 = grp * 64;
     const bool active = r0 < t.rows_pad;
     const int r = active ? r0 + lane : lane;
-    (void)eng_prologue<NW, eng_norm_segs<NW, kQ8_0, MULTI>()>(a, L, 0, t.cols, [] {});
+    (void)eng_prologue<NW, eng_norm_segs<NW, kQ8_0, false>()>(a, L, 0, t.cols, [] {});
     if (!active) return;
     const float sc = L.red[1];
     float sum = 0.0f;
@@ -3265,7 +3265,7 @@ __device__ __forceinline__ void eng_dispatch(const TmqEngAct& a, const EngLds& L
     else if constexpr (FMT == kQ8_DIRECT) eng_group_q8<NW>(a, L, w, g);
     else if constexpr (FMT == kI16) eng_group_i16_split<NW, MULTI>(a, L, w, g);
     else if constexpr (FMT == kI16_DIRECT) eng_group_i16<NW>(a, L, w, g);
-    else if constexpr (FMT == kF32P) eng_group_f32<NW, MULTI>(a, L, w, g);
+    else if constexpr (FMT == kF32P) eng_group_f32<NW>(a, L, w, g);
     else if constexpr (FMT == kF32R) eng_group_f32_rows<NW, MULTI>(a, L, w, g);
     else if constexpr (FMT == kQ5_0M || FMT == kQ4_KM || FMT == kQ6_KM) eng_group_mfma<FMT, NW, MULTI>(a, L, w, g);
     else eng_group_k<FMT, NW, MULTI>(a, L, w, g);
@@ -3332,7 +3332,6 @@ __global__ __launch_bounds__(256) void resid_view_kernel(const float* __restrict
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) out[i] = x[i] + tmq_fin(d, i);
 }
 
-// Zeroes n int64 K-split accumulators (at the device coherence point).
 // The rows of a tiled product (Q8_0, INT16), finalised once: the fold of
 // tmq_fin with the tiles' loads 16 at a time.  Left to the next launch, every
 // one of its workgroups folds all rows in its prologue (76 tiles of 896 rows:
@@ -3355,6 +3354,7 @@ __global__ __launch_bounds__(64) void fin_tiles_kernel(TmqDeferred d, int n, flo
         __hip_atomic_store(out + i, y, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// Zeroes n int64 K-split accumulators (at the device coherence point).
 __global__ __launch_bounds__(256) void zero_acc_kernel(int64_t* p, size_t n) {
     for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
         __hip_atomic_store(p + i, (int64_t)0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -4287,7 +4287,7 @@ static int f32_rows_max(const TmqTensorDev& t) {
     const bool f32 = t.type == kF32;
     if (t.cols < (f32 ? 160 : 128)) return 0;
     const int per = f32 ? 32 : t.type == kF16 || t.type == kQ8_0 ? 48 : 60;
-    return (int)std::min<int64_t>(f32 ? 24576 : TMQ_F32_ROWS_MAX, (int64_t)per * t.cols);
+    return (int)std::min<int64_t>(f32 ? 24576 : 65536, (int64_t)per * t.cols);
 }
 int tmq_launch_gemv(const TmqWork& w, hipStream_t s) {
     if (w.ngroups <= 0) return 0;
@@ -4458,13 +4458,13 @@ static void* eng_kernel_for(int fa, int fb) {
     if constexpr (NW == 4) {
         // the INT16 / FP32 branches (4-wave launches only)
         if (fa == kI16 && fb == kI16) return TMQ_ENG_K(kI16, kI16);
-        if (fa == kF32P && fb == kF32P) return TMQ_ENG_K(kF32P, kF32P);
         if (fa == kF32R && fb == kF32R) return TMQ_ENG_K(kF32R, kF32R);
         if constexpr (MULTI) {
             if (fa == kQ5_0 && fb == kI16) return TMQ_ENG_K(kQ5_0, kI16);
             if (fa == kI16 && fb == kQ8_0) return TMQ_ENG_K(kI16, kQ8_0);
         } else {
             if (fa == kI16_DIRECT && fb == kI16_DIRECT) return TMQ_ENG_K(kI16_DIRECT, kI16_DIRECT);
+            if (fa == kF32P && fb == kF32P) return TMQ_ENG_K(kF32P, kF32P);
         }
     }
 #undef TMQ_ENG_K
@@ -4479,7 +4479,7 @@ static int eng_resolve(const TmqEngLaunch& l, int waves, void** kernel, size_t* 
     // format of the first and the last work (the others must match the first)
     auto code = [](const TmqWork& w) {
         if (w.path == TMQ_WPATH_INT16) return w.kacc ? kI16 : kI16_DIRECT;
-        if (w.path == TMQ_WPATH_FP32) return w.cand || w.t.rows > TMQ_F32_ROWS_MAX ? kF32P : kF32R;
+        if (w.path == TMQ_WPATH_FP32) return w.cand ? kF32P : kF32R;
         if (w.t.type == kQ8_0) return w.kacc ? kQ8_0 : kQ8_DIRECT;
         // the MFMA decoders where the tensor carries their planes
         return tmq_kernel_fmt(w.t);

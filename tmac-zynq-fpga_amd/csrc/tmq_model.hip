@@ -862,7 +862,7 @@ int build_launches(tmq_model* m) {
         if (w.path == TMQ_WPATH_FP32) {
             w.kc = 1;
             w.y = (float*)kacc;
-            w.ngroups = t->dev.rows > TMQ_F32_ROWS_MAX ? (g64 + ln.waves - 1) / ln.waves : t->dev.rows_pad / TMQ_F32_ROWS;
+            w.ngroups = t->dev.rows_pad / TMQ_F32_ROWS;
         } else {
             // (the MFMA decoders split a row by whole blocks / super-blocks)
             const int units = (t->dev.type == TMQ_TYPE_Q8_0 || w.path == TMQ_WPATH_INT16) ? (t->dev.cols + 63) / 64

@@ -634,13 +634,13 @@ __global__ __launch_bounds__(256, TILE == 1 ? 2 : TILE == 3 ? 3 : 1) void pf_gem
 template <int MODE>
 __global__ __launch_bounds__(256, MODE == TMQ_PF_QKV ? 1 : 2) void pf_gemm_few_kernel(TmqPfGemm g) {
     tmq_warm_kernargs<sizeof(TmqPfGemm)>();
-    constexpr int R = 4, NTB = 1;
+    constexpr int R = 4;
     __shared__ int red[4][3 * 16][64];  // (a row block at a time: two workgroups a CU)
     __shared__ uint64_t c_tab[32];
     __shared__ float smax[4][32];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    const int bx = blockIdx.x, bz = blockIdx.z, tb0 = blockIdx.y * NTB;
+    const int bx = blockIdx.x, bz = blockIdx.z, tb = blockIdx.y;
     auto rblk = [&](int i) -> int { return MODE == TMQ_PF_GU ? i * (g.gu_rows >> 5) + bx : 2 * bx + i; };
     // whole 64-column tiles a wave (the Q8_0 sums are per tile)
     const int nks = g.K >> 5, nt = g.K >> 6;
@@ -659,9 +659,9 @@ __global__ __launch_bounds__(256, MODE == TMQ_PF_QKV ? 1 : 2) void pf_gemm_few_k
     const int r4 = 8 * wave + 4 * (lane >> 5);
     float4 inv4[2], bias4[2];
     int4 rw4[2];
-    float4 cs4[NTB][2];
-    float xs_raw[NTB];
-    int32_t tx_raw[NTB];
+    float4 cs4[2];
+    float xs_raw = 0.0f;
+    int32_t tx_raw = 0;
     const bool hasb = MODE == TMQ_PF_QKV && S.bias != nullptr;
     if (MODE != TMQ_PF_PART && !q8) {
 #pragma unroll
@@ -671,22 +671,17 @@ __global__ __launch_bounds__(256, MODE == TMQ_PF_QKV ? 1 : 2) void pf_gemm_few_k
             inv4[i] = *(const float4*)(Sg.row_inv + rr);
             rw4[i] = *(const int4*)(g.rw_t + row);
             if (hasb) bias4[i] = *(const float4*)(Sg.bias + rr);
-#pragma unroll
-            for (int j = 0; j < NTB; j++)
-                if (MODE == TMQ_PF_QKV && si != 2)
-                    cs4[j][i] = *(const float4*)(g.rope + (size_t)(g.p0 + min((tb0 + j) * 32 + (lane & 31), g.T - 1)) * 32 +
-                                                 ((rr & 63) >> 1));
+            if (MODE == TMQ_PF_QKV && si != 2)
+                cs4[i] = *(const float4*)(g.rope + (size_t)(g.p0 + min(tb * 32 + (lane & 31), g.T - 1)) * 32 +
+                                         ((rr & 63) >> 1));
         }
-#pragma unroll
-        for (int j = 0; j < NTB; j++) {
-            xs_raw[j] = g.xs[(tb0 + j) * 32 + (lane & 31)];
-            tx_raw[j] = g.tx_t[(tb0 + j) * 32 + (lane & 31)];
-        }
+        xs_raw = g.xs[tb * 32 + (lane & 31)];
+        tx_raw = g.tx_t[tb * 32 + (lane & 31)];
     }
     if (MODE == TMQ_PF_GU && threadIdx.x < 32) c_tab[threadIdx.x] = tmq_math::exp2_tab(threadIdx.x);
 
     struct Step {
-        tmq_v4i w[2][2], x[NTB][2];
+        tmq_v4i w[2][2], x[2];
     } st[R];
     // column step s (steps past the wave's last re-read it)
     auto load = [&](Step& k, int s) {
@@ -696,18 +691,14 @@ __global__ __launch_bounds__(256, MODE == TMQ_PF_QKV ? 1 : 2) void pf_gemm_few_k
 #pragma unroll
             for (int i = 0; i < 2; i++)
                 k.w[i][d] = *(const tmq_v4i*)(g.w + (((size_t)rblk(i) * nks + s) * 2 + d) * 1024 + lane * 16);
-#pragma unroll
-            for (int j = 0; j < NTB; j++)
-                k.x[j][d] = *(const tmq_v4i*)(g.x + (((size_t)(tb0 + j) * nks + s) * 2 + d) * 1024 + lane * 16);
+            k.x[d] = *(const tmq_v4i*)(g.x + (((size_t)tb * nks + s) * 2 + d) * 1024 + lane * 16);
         }
     };
-    tmq_v16i acc[2][NTB][3];
+    tmq_v16i acc[2][3];
 #pragma unroll
     for (int i = 0; i < 2; i++)
 #pragma unroll
-        for (int j = 0; j < NTB; j++)
-#pragma unroll
-            for (int d = 0; d < 3; d++) acc[i][j][d] = tmq_v16i{};
+        for (int d = 0; d < 3; d++) acc[i][d] = tmq_v16i{};
     static_for<R>([&](auto bc) { load(st[decltype(bc)::value], s0 + decltype(bc)::value); });
     auto kloop = [&](auto q8c) {
         constexpr bool Q8 = decltype(q8c)::value;
@@ -717,31 +708,26 @@ __global__ __launch_bounds__(256, MODE == TMQ_PF_QKV ? 1 : 2) void pf_gemm_few_k
                 Step& k = st[b];
                 if (sb + b < s1) {
 #pragma unroll
-                    for (int j = 0; j < NTB; j++)
-#pragma unroll
-                        for (int i = 0; i < 2; i++) {
-                            acc[i][j][0] = mfma(k.w[i][0], k.x[j][0], acc[i][j][0]);
-                            acc[i][j][1] = mfma(k.w[i][0], k.x[j][1], acc[i][j][1]);
-                            acc[i][j][2] = mfma(k.w[i][1], k.x[j][1], acc[i][j][2]);
-                            acc[i][j][1] = mfma(k.w[i][1], k.x[j][0], acc[i][j][1]);
-                        }
+                    for (int i = 0; i < 2; i++) {
+                        acc[i][0] = mfma(k.w[i][0], k.x[0], acc[i][0]);
+                        acc[i][1] = mfma(k.w[i][0], k.x[1], acc[i][1]);
+                        acc[i][2] = mfma(k.w[i][1], k.x[1], acc[i][2]);
+                        acc[i][1] = mfma(k.w[i][1], k.x[0], acc[i][1]);
+                    }
                     if (Q8 && (b & 1)) {
                         // the 64-column tile just completed (R and s0 even)
                         const int tile = (sb + b) >> 1;
+                        const int t = tb * 32 + (lane & 31);
 #pragma unroll
-                        for (int j = 0; j < NTB; j++) {
-                            const int t = (tb0 + j) * 32 + (lane & 31);
+                        for (int i = 0; i < 2; i++) {
+                            int64_t* out = g.tpart + ((size_t)tile * S.rows + rblk(i) * 32 - S.row0) * g.T_pad + t;
 #pragma unroll
-                            for (int i = 0; i < 2; i++) {
-                                int64_t* out = g.tpart + ((size_t)tile * S.rows + rblk(i) * 32 - S.row0) * g.T_pad + t;
+                            for (int v = 0; v < 16; v++)
+                                out[(size_t)blk_row(v, lane) * g.T_pad] = 65536 * (int64_t)acc[i][0][v] +
+                                                                           256 * (int64_t)acc[i][1][v] +
+                                                                           (int64_t)acc[i][2][v];
 #pragma unroll
-                                for (int v = 0; v < 16; v++)
-                                    out[(size_t)blk_row(v, lane) * g.T_pad] = 65536 * (int64_t)acc[i][j][0][v] +
-                                                                               256 * (int64_t)acc[i][j][1][v] +
-                                                                               (int64_t)acc[i][j][2][v];
-#pragma unroll
-                                for (int d = 0; d < 3; d++) acc[i][j][d] = tmq_v16i{};
-                            }
+                            for (int d = 0; d < 3; d++) acc[i][d] = tmq_v16i{};
                         }
                     }
                 }
@@ -754,93 +740,90 @@ __global__ __launch_bounds__(256, MODE == TMQ_PF_QKV ? 1 : 2) void pf_gemm_few_k
     }
     kloop(std::integral_constant<bool, false>{});
 
+    int sum[2][3][4];
 #pragma unroll
-    for (int j = 0; j < NTB; j++) {
-        int sum[2][3][4];
+    for (int i = 0; i < 2; i++) {
+        if (i) __syncthreads();  // the first block's sums are read
 #pragma unroll
-        for (int i = 0; i < 2; i++) {
-            if (i) __syncthreads();  // the first block's sums are read
+        for (int d = 0; d < 3; d++)
 #pragma unroll
-            for (int d = 0; d < 3; d++)
+            for (int v = 0; v < 16; v++) red[wave][d * 16 + v][lane] = acc[i][d][v];
+        __syncthreads();
 #pragma unroll
-                for (int v = 0; v < 16; v++) red[wave][d * 16 + v][lane] = acc[i][j][d][v];
-            __syncthreads();
-#pragma unroll
-            for (int d = 0; d < 3; d++)
-#pragma unroll
-                for (int k = 0; k < 4; k++) {
-                    const int e = d * 16 + 4 * wave + k;
-                    sum[i][d][k] = red[0][e][lane] + red[1][e][lane] + red[2][e][lane] + red[3][e][lane];
-                }
-        }
-        const int t = (tb0 + j) * 32 + (lane & 31);
-        const bool live = t < g.T;
-        if (MODE == TMQ_PF_PART) {
-            if (!live) continue;
-#pragma unroll
-            for (int i = 0; i < 2; i++) {
-                int64_t o[4];
-#pragma unroll
-                for (int k = 0; k < 4; k++)
-                    o[k] = 65536 * (int64_t)sum[i][0][k] + 256 * (int64_t)sum[i][1][k] + (int64_t)sum[i][2][k];
-                int64_t* dst = g.part + ((size_t)bz * g.T_pad + t) * g.rows + rblk(i) * 32 + r4;
-                *(longlong2*)dst = longlong2{o[0], o[1]};
-                *(longlong2*)(dst + 2) = longlong2{o[2], o[3]};
-            }
-            continue;
-        }
-        // finalised as in pf_gemm_kernel (sim/tmac_gguf.cpp:1303-1305)
-        const double xs = (double)xs_raw[j], tc = (double)(128 * (int64_t)tx_raw[j] + 16384 * (int64_t)g.K);
-        float o[2][4];
-#pragma unroll
-        for (int i = 0; i < 2; i++) {
-            const float iv[4] = {inv4[i].x, inv4[i].y, inv4[i].z, inv4[i].w};
-            const int rw[4] = {rw4[i].x, rw4[i].y, rw4[i].z, rw4[i].w};
-            const float bv[4] = {bias4[i].x, bias4[i].y, bias4[i].z, bias4[i].w};
+        for (int d = 0; d < 3; d++)
 #pragma unroll
             for (int k = 0; k < 4; k++) {
-                const double a = digits_f64(sum[i][0][k], sum[i][1][k], sum[i][2][k], tc + (double)(128 * rw[k]));
-                o[i][k] = (float)((a * xs) / (double)iv[k]);
-                if (hasb) o[i][k] = o[i][k] + bv[k];
+                const int e = d * 16 + 4 * wave + k;
+                sum[i][d][k] = red[0][e][lane] + red[1][e][lane] + red[2][e][lane] + red[3][e][lane];
             }
-        }
-        if (MODE == TMQ_PF_QKV) {
-            if (!live) continue;
+    }
+    const int t = tb * 32 + (lane & 31);
+    const bool live = t < g.T;
+    if (MODE == TMQ_PF_PART) {
+        if (!live) return;
 #pragma unroll
-            for (int i = 0; i < 2; i++) {
-                const int rr = rblk(i) * 32 + r4 - S.row0;
-                if (si != 2) {
-                    // apply_rope (sim/tmac_gguf.cpp:1537-1539)
-                    const float4 cs = cs4[j][i];
-                    const float a = o[i][0], b = o[i][1], c = o[i][2], d = o[i][3];
-                    o[i][0] = a * cs.x - b * cs.y;
-                    o[i][1] = a * cs.y + b * cs.x;
-                    o[i][2] = c * cs.z - d * cs.w;
-                    o[i][3] = c * cs.w + d * cs.z;
-                }
-                float* dst = si == 0   ? g.q_out + (size_t)t * g.H + rr
-                             : si == 1 ? g.kc + (size_t)(g.p0 + t) * g.KV + rr
-                                       : g.vc + (size_t)(g.p0 + t) * g.KV + rr;
-                *(float4*)dst = make_float4(o[i][0], o[i][1], o[i][2], o[i][3]);
-            }
-        } else {
-            // SwiGLU (:459-461) and the token's largest |value| in this workgroup
-            float s[4], m = 0.0f;
+        for (int i = 0; i < 2; i++) {
+            int64_t o[4];
 #pragma unroll
-            for (int k = 0; k < 4; k++) {
-                s[k] = (o[0][k] / (1.0f + tmq_math::tmq_expf_tab(-o[0][k], Exp2TabLds{c_tab}))) * o[1][k];
-                m = fmaxf(m, fabsf(s[k]));
-            }
-            if (live) *(float4*)(g.s_out + (size_t)t * g.gu_rows + bx * 32 + r4) = make_float4(s[0], s[1], s[2], s[3]);
-            m = fmaxf(m, __shfl_xor(m, 32));
-            if (lane < 32) smax[wave][lane] = m;
-            __syncthreads();
-            if (wave == 0 && live && lane < 32)
-                __hip_atomic_fetch_max(g.max_bits + t,
-                                       __builtin_bit_cast(uint32_t, fmaxf(fmaxf(smax[0][lane], smax[1][lane]),
-                                                                          fmaxf(smax[2][lane], smax[3][lane]))),
-                                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            for (int k = 0; k < 4; k++)
+                o[k] = 65536 * (int64_t)sum[i][0][k] + 256 * (int64_t)sum[i][1][k] + (int64_t)sum[i][2][k];
+            int64_t* dst = g.part + ((size_t)bz * g.T_pad + t) * g.rows + rblk(i) * 32 + r4;
+            *(longlong2*)dst = longlong2{o[0], o[1]};
+            *(longlong2*)(dst + 2) = longlong2{o[2], o[3]};
         }
+        return;
+    }
+    // finalised as in pf_gemm_kernel (sim/tmac_gguf.cpp:1303-1305)
+    const double xs = (double)xs_raw, tc = (double)(128 * (int64_t)tx_raw + 16384 * (int64_t)g.K);
+    float o[2][4];
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        const float iv[4] = {inv4[i].x, inv4[i].y, inv4[i].z, inv4[i].w};
+        const int rw[4] = {rw4[i].x, rw4[i].y, rw4[i].z, rw4[i].w};
+        const float bv[4] = {bias4[i].x, bias4[i].y, bias4[i].z, bias4[i].w};
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const double a = digits_f64(sum[i][0][k], sum[i][1][k], sum[i][2][k], tc + (double)(128 * rw[k]));
+            o[i][k] = (float)((a * xs) / (double)iv[k]);
+            if (hasb) o[i][k] = o[i][k] + bv[k];
+        }
+    }
+    if (MODE == TMQ_PF_QKV) {
+        if (!live) return;
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            const int rr = rblk(i) * 32 + r4 - S.row0;
+            if (si != 2) {
+                // apply_rope (sim/tmac_gguf.cpp:1537-1539)
+                const float4 cs = cs4[i];
+                const float a = o[i][0], b = o[i][1], c = o[i][2], d = o[i][3];
+                o[i][0] = a * cs.x - b * cs.y;
+                o[i][1] = a * cs.y + b * cs.x;
+                o[i][2] = c * cs.z - d * cs.w;
+                o[i][3] = c * cs.w + d * cs.z;
+            }
+            float* dst = si == 0   ? g.q_out + (size_t)t * g.H + rr
+                         : si == 1 ? g.kc + (size_t)(g.p0 + t) * g.KV + rr
+                                   : g.vc + (size_t)(g.p0 + t) * g.KV + rr;
+            *(float4*)dst = make_float4(o[i][0], o[i][1], o[i][2], o[i][3]);
+        }
+    } else {
+        // SwiGLU (:459-461) and the token's largest |value| in this workgroup
+        float s[4], m = 0.0f;
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            s[k] = (o[0][k] / (1.0f + tmq_math::tmq_expf_tab(-o[0][k], Exp2TabLds{c_tab}))) * o[1][k];
+            m = fmaxf(m, fabsf(s[k]));
+        }
+        if (live) *(float4*)(g.s_out + (size_t)t * g.gu_rows + bx * 32 + r4) = make_float4(s[0], s[1], s[2], s[3]);
+        m = fmaxf(m, __shfl_xor(m, 32));
+        if (lane < 32) smax[wave][lane] = m;
+        __syncthreads();
+        if (wave == 0 && live && lane < 32)
+            __hip_atomic_fetch_max(g.max_bits + t,
+                                   __builtin_bit_cast(uint32_t, fmaxf(fmaxf(smax[0][lane], smax[1][lane]),
+                                                                      fmaxf(smax[2][lane], smax[3][lane]))),
+                                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
 }
 
