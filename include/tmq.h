@@ -253,8 +253,9 @@ int tmq_phaseb_run(tmq_ctx* ctx, uint8_t* arena, uint64_t arena_bytes, uint32_t 
  * descriptor chain built by phaseb_add_descriptor (sim/tmac_gguf.cpp:533-574).
  * num_tiles/tile_res_rows/num_col_groups keep the PhaseB meaning: output rows
  * = num_tiles*tile_res_rows (Q5_0, Q8_0) or (num_tiles/num_col_groups)*
- * tile_res_rows (Q4_K, Q6_K), and must match the tensor.  All descriptors run
- * in one kernel launch (plus one activation-quantisation launch). */
+ * tile_res_rows (Q4_K, Q6_K), and must match the tensor.  All descriptors of
+ * a format run in one kernel launch, after one activation-quantisation launch;
+ * a small chain's run is one launch altogether. */
 typedef struct {
     const tmq_tensor* weight;
     const float* x_dev;   /* fp32 activation, device */
@@ -266,8 +267,9 @@ typedef struct {
 } tmq_desc;
 
 int tmq_chain_create(tmq_ctx* ctx, const tmq_desc* descs, int n, tmq_chain** out);
-/* tmq_chain_run = tmq_chain_prepare (quantise the chain's activations, one
- * launch) + tmq_chain_launch (all matmul descriptors, one launch).  The two
+/* tmq_chain_run does what tmq_chain_prepare (quantise the chain's activations,
+ * one launch) and tmq_chain_launch (all matmul descriptors, a launch a format)
+ * do, and leaves the prepared activations as tmq_chain_prepare does.  The two
  * halves are exposed so a caller can re-run the matmuls on activations that
  * have not changed. */
 int tmq_chain_run(tmq_ctx* ctx, tmq_chain* chain);
